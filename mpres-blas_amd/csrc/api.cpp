@@ -121,6 +121,7 @@ struct mpres_ctx {
     int *dpow2 = nullptr;
     int bits = 0;  // bit length of the largest modulus
     const Ops *ops[OP_COUNT] = {};
+    const PosOps *pos = nullptr;  // positional reductions (8 moduli)
     // per operation, an optional table of lane counts by call size (mpres_set_lanes_table):
     // entry i serves calls of size <= bound[i], the last entry larger ones
     struct LanesTable {
@@ -219,6 +220,15 @@ struct WsUse {
         pool = true;
         *out = (char *)c->ws;
         return MPRES_OK;
+    }
+    // as get, for a call that runs faster with `full` bytes but does with `need`: *have tells
+    // whether there are `full` (a caller's smaller workspace, or a pool that cannot grow so far,
+    // is taken as it is)
+    int get2(void *ws, size_t ws_bytes, size_t need, size_t full, char **out, bool *have) {
+        *have = full > need && (ws ? ws_bytes >= full : get(nullptr, 0, full, out) == MPRES_OK);
+        if (*have && !ws) return MPRES_OK;
+        if (!ws) (void)hipGetLastError();
+        return get(ws, ws_bytes, need, out);
     }
     ~WsUse() {
         if (!pool) return;
@@ -347,6 +357,7 @@ int mpres_ctx_create(mpres_ctx_t **out, int set_id, int device) {
         }
         install_builtin_lanes(c, op);
     }
+    c->pos = pos_ops(s->n);
     if (hipMalloc(&c->dpow2, pow2.size() * sizeof(int)) != hipSuccess ||
         hipMalloc(&c->dev, sizeof(DevConsts)) != hipSuccess) {
         (void)hipFree(c->dpow2);
@@ -648,6 +659,10 @@ size_t mpres_dot_workspace(const mpres_ctx_t *c, int n, int g3, int b3) {
     return mpsize(c) * ((size_t)g3 * b3 + (size_t)g3 + (size_t)b3 + 1);
 }
 
+// Terms per chain from which the positional chains are used: converting a sum back and evaluating
+// it costs about as much as 6 terms of the residue chain (8 moduli, 256 x 64 chains: 4 terms
+// 31 us against 23 us, 16 terms about 50 us against 95 us, 1024 terms 1.50 ms against 6.12 ms).
+constexpr long long POS_DOT_TERMS = 8;
 static int dot_common(mpres_ctx_t *c, WsUse &wu, int mode, int n, SoA xs, int incx, SoA ys, int incy,
                       const char *xa, const char *ya, int g3, int b3, void *ws, size_t wsb, hipStream_t st,
                       char **result) {
@@ -659,12 +674,16 @@ static int dot_common(mpres_ctx_t *c, WsUse &wu, int mode, int n, SoA xs, int in
     char *p1 = w, *p2 = p1 + S * G, *p3 = p2 + S * g3, *p4 = p3 + S * b3;
     const Ops *o = sized(c, OP_DOT, n);
     const unsigned P = next_pow2((unsigned)b3);
+    const bool pos = c->pos && n >= POS_DOT_TERMS * G;
     // pass 1: strided fold over the products, halving tree per block of b3 (src/mpreduct.cuh:38-74)
     {
         ProfScope ps(c, OP_DOT, st);
-        HIPCHK(o->fold(c->dev, mode, 0, n, G, xs, incx, ys, incy, xa, ya, p1, st));
+        if (pos)
+            HIPCHK(c->pos->fold(c->dev, mode, n, G, xs, incx, ys, incy, xa, ya, p1, st));
+        else
+            HIPCHK(o->fold(c->dev, mode, 0, n, G, xs, incx, ys, incy, xa, ya, p1, st));
     }
-    HIPCHK(o->fold(c->dev, mode, 1, n, G, xs, incx, ys, incy, xa, ya, p1, st));
+    if (pos || c->host.n > 8) HIPCHK(o->fold(c->dev, mode, 1, n, G, xs, incx, ys, incy, xa, ya, p1, st));
     HIPCHK(o->tree(c->dev, p1, b3, P, g3, p2, st));
     // pass 2: one block of b3 over the g3 block results (src/mpreduct.cuh:81-112)
     SoA none{};
@@ -899,12 +918,18 @@ int mpres_dsqrt(mpres_ctx_t *c, int count, const void *x, double *out, void *st)
 }
 
 // ---------------------------------------------------------------- gemv
+// alpha*x, the ly*b3 partials, the ly row sums, then the main kernel's auxiliary data; after
+// it (mpres_gemv_workspace) the positional kernel's records of alpha*x, which a smaller
+// workspace goes without
+static size_t gemv_need(const mpres_ctx_t *c, bool tr, int m, int n, int b3) {
+    const size_t lx = tr ? m : n, ly = tr ? n : m;
+    return mpsize(c) * (lx + ly * (size_t)b3 + ly) + c->ops[OP_GEMV]->gemv_aux(tr, m, n);
+}
 size_t mpres_gemv_workspace(const mpres_ctx_t *c, int trans, int m, int n, int b3) {
     if (!c || m <= 0 || n <= 0 || b3 <= 0) return 0;
     const bool tr = trans != MPRES_NO_TRANS;
-    const size_t lx = tr ? m : n, ly = tr ? n : m;
-    // alpha*x, the ly*b3 partials, the ly row sums, then the main kernel's auxiliary data
-    return mpsize(c) * (lx + ly * (size_t)b3 + ly) + c->ops[OP_GEMV]->gemv_aux(tr, m, n);
+    const size_t lx = tr ? m : n;
+    return gemv_need(c, tr, m, n, b3) + (c->pos ? 16 + c->pos->rec_bytes((long long)lx) : 0);
 }
 
 int mpres_gemv(mpres_ctx_t *c, int trans, int m, int n, const mp_array_t *alpha, const mp_array_t *A, int lda,
@@ -922,8 +947,11 @@ int mpres_gemv(mpres_ctx_t *c, int trans, int m, int n, const mp_array_t *alpha,
     const size_t S = mpsize(c);
     char *w;
     WsUse wu(c, strm(st));
-    int rc = wu.get(ws, wsb, mpres_gemv_workspace(c, trans, m, n, b3), &w);
+    bool full;
+    const size_t need = gemv_need(c, tr, m, n, b3);
+    int rc = wu.get2(ws, wsb, need, mpres_gemv_workspace(c, trans, m, n, b3), &w, &full);
     if (rc) return rc;
+    char *rec = full ? w + (need + 15) / 16 * 16 : nullptr;
     char *bx = w, *part = bx + S * lx, *sums = part + S * (size_t)ly * b3, *aux = sums + S * (size_t)ly;
     const Ops *o = sized(c, OP_GEMV, (long long)m * n);
     SoA ys = soa_of(y);
@@ -944,21 +972,33 @@ int mpres_gemv(mpres_ctx_t *c, int trans, int m, int n, const mp_array_t *alpha,
         }
         HIPCHK(o->gemv_fold(c->dev, tr, 2, m, n, soa_of(A), lda, bx, b3, nvt, part, aux, strm(st)));
         HIPCHK(fk.join());
-    } else {
+    } else if (c->host.n > 8) {
         ProfScope ps(c, OP_GEMV, strm(st));
         HIPCHK(o->gemv_fold(c->dev, tr, 1, m, n, soa_of(A), lda, bx, b3, nvt, part, aux, strm(st)));
     }
     HIPCHK(o->gemv_fold(c->dev, tr, 3, m, n, soa_of(A), lda, bx, b3, nvt, part, aux, strm(st)));
+    if (c->pos) {
+        if (rec) HIPCHK(c->pos->records(c->dev, 0, 0, lx, 1, SoA{}, bx, false, lx, rec, strm(st)));
+        ProfScope ps(c, c->host.n > 8 ? -1 : (int)OP_GEMV, strm(st));
+        HIPCHK(c->pos->gemv(c->dev, tr, m, n, soa_of(A), lda, bx, rec, b3, nvt, part, strm(st)));
+    }
+    HIPCHK(o->gemv_fold(c->dev, tr, 4, m, n, soa_of(A), lda, bx, b3, nvt, part, aux, strm(st)));
     HIPCHK(o->tree(c->dev, part, b3, next_pow2((unsigned)b3), ly, sums, strm(st)));
     HIPCHK(o->gemv_final(c->dev, ly, ys, incy, sums, strm(st)));
     return MPRES_OK;
 }
 
 // ---------------------------------------------------------------- gemm
+// the m*n dot-product sums, and over 16/32 moduli the pre-scaled residue planes; after them
+// (mpres_gemm_workspace) the positional kernel's records of A and B, which a smaller workspace
+// goes without
+static size_t gemm_need(const mpres_ctx_t *c, int m, int n, int k) { return c->ops[OP_GEMM]->gemm_ws(m, n, k); }
+static size_t gemm_rec_bytes(const mpres_ctx_t *c, int cnt, int k) {
+    return (c->pos->rec_bytes((long long)cnt * k) + 255) / 256 * 256;
+}
 size_t mpres_gemm_workspace(const mpres_ctx_t *c, int m, int n, int k) {
     if (!c || m <= 0 || n <= 0 || k < 0) return 0;
-    // the m*n dot-product sums, and over 16/32 moduli the pre-scaled residue planes
-    return c->ops[OP_GEMM]->gemm_ws(m, n, k);
+    return gemm_need(c, m, n, k) + (c->pos ? 256 + gemm_rec_bytes(c, m, k) + gemm_rec_bytes(c, n, k) : 0);
 }
 
 int mpres_gemm(mpres_ctx_t *c, int ta, int tb, int m, int n, int k, const mp_array_t *alpha, const mp_array_t *A,
@@ -976,9 +1016,26 @@ int mpres_gemm(mpres_ctx_t *c, int ta, int tb, int m, int n, int k, const mp_arr
         return fail(MPRES_ERR_ARG, "digits of A and B must be 16-byte aligned");
     char *w;
     WsUse wu(c, strm(st));
-    int rc = wu.get(ws, wsb, mpres_gemm_workspace(c, m, n, k), &w);
+    bool full;
+    const size_t need = gemm_need(c, m, n, k);
+    int rc = wu.get2(ws, wsb, need, mpres_gemm_workspace(c, m, n, k), &w, &full);
     if (rc) return rc;
+    char *ra = full ? w + (need + 255) / 256 * 256 : nullptr, *rb = full ? ra + gemm_rec_bytes(c, m, k) : nullptr;
     const Ops *o = sized(c, OP_GEMM, (long long)m * n * k);
+    if (c->host.n == 8) {
+        if (full) {
+            HIPCHK(c->pos->records(c->dev, 0, 0, m, k, soa_of(A), nullptr, true, lda, ra, strm(st)));
+            HIPCHK(c->pos->records(c->dev, 1, 0, n, k, soa_of(B), nullptr, true, ldb, rb, strm(st)));
+        }
+        {
+            ProfScope ps(c, OP_GEMM, strm(st));
+            HIPCHK(c->pos->gemm(c->dev, 0, 0, m, n, k, soa_of(A), lda, soa_of(B), ldb, ra, rb, w, strm(st)));
+        }
+        for (int pass = 3; pass < 5; pass++)
+            HIPCHK(o->gemm(c->dev, pass, c->bits, m, n, k, soa_of(alpha), soa_of(A), lda, soa_of(B), ldb, soa_of(beta),
+                           soa_of(C), ldc, w, strm(st)));
+        return MPRES_OK;
+    }
     // the residue path (pass 0) runs on the side stream while the chains (pass 1) run on st
     Fork fk(c, strm(st));
     {
@@ -1031,14 +1088,24 @@ int mpres_gemm_v2(mpres_ctx_t *c, int ta, int tb, int m, int n, int k, const voi
     if (k < 0 || lda <= 0 || ldb <= 0 || ldc < std::max(1, m)) return fail(MPRES_ERR_ARG, "invalid dimensions");
     char *w;
     WsUse wu(c, strm(st));
-    int rc = wu.get(ws, wsb, mpres_gemm_workspace(c, m, n, k), &w);
+    bool full;
+    const size_t need = gemm_need(c, m, n, k);
+    int rc = wu.get2(ws, wsb, need, mpres_gemm_workspace(c, m, n, k), &w, &full);
     if (rc) return rc;
+    char *ra = full ? w + (need + 255) / 256 * 256 : nullptr, *rb = full ? ra + gemm_rec_bytes(c, m, k) : nullptr;
     const int tra = ta == MPRES_TRANS || ta == MPRES_CONJ_TRANS, trb = tb == MPRES_TRANS || tb == MPRES_CONJ_TRANS;
     // as in mpres_gemm: the residue path (pass 0) on the side stream, the chains on st
     const Ops *o = sized(c, OP_GEMM, (long long)m * n * k);
     Fork fk(c, strm(st));
+    if (full) {
+        HIPCHK(c->pos->records(c->dev, 0, tra, m, k, SoA{}, (const char *)A, false, lda, ra, fk.s1));
+        HIPCHK(c->pos->records(c->dev, 1, trb, n, k, SoA{}, (const char *)B, false, ldb, rb, fk.s1));
+    }
     for (int pass = 0; pass < 5; pass++) {
         if (pass == 2) HIPCHK(fk.join());
+        if (pass == 3 && c->pos)
+            HIPCHK(c->pos->gemm_v2(c->dev, tra, trb, m, n, k, (const char *)A, lda, (const char *)B, ldb, ra, rb, w,
+                                   strm(st)));
         HIPCHK(o->gemm_v2(c->dev, pass, c->bits, tra, trb, m, n, k, (const char *)alpha, (const char *)A,
                                         lda, (const char *)B, ldb, (const char *)beta, (char *)C, ldc, w,
                                         pass == 0 ? fk.s1 : strm(st)));

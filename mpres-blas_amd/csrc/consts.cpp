@@ -168,6 +168,32 @@ bool compute_consts(const ModuliSet &s, DevConsts &c, std::vector<int> &pow2) {
         c.rrd[i] = emu_div_rd(1.0, (double)s.m[i]);
         c.rru[i] = emu_div_ru(1.0, (double)s.m[i]);
     }
+    // limbs of M and of M / m_i, powers of 2^16 modulo m_i
+    {
+        const auto limb16 = [](const std::vector<uint32_t> &v, int l) {
+            return l / 2 < (int)v.size() ? (double)((v[l / 2] >> (16 * (l & 1))) & 0xffffu) : 0.0;
+        };
+        double pm = 0;
+        for (size_t i = M.size(); i-- > 0;) pm = pm * 4294967296.0 + (double)M[i];
+        c.pmod = pm;
+        c.pinv = 1.0 / pm;
+        for (int l = 0; l < 2 * n; l++) c.m16[l] = limb16(M, l);
+        for (int j = 0; j < n; j++) {
+            std::vector<uint32_t> Q(M);
+            uint64_t rem = 0;
+            for (size_t i = Q.size(); i-- > 0;) {
+                const uint64_t t = (rem << 32) | Q[i];
+                Q[i] = (uint32_t)(t / (uint32_t)s.m[j]);
+                rem = t % (uint32_t)s.m[j];
+            }
+            int64_t q = 1;
+            for (int l = 0; l < 2 * n; l++) {
+                c.mi16[l][j] = limb16(Q, l);
+                c.q16[l][j] = (double)q;
+                q = (q << 16) % s.m[j];
+            }
+        }
+    }
     // MP_PRECISION, MP_H, MP_J from b = floor(log2 M53) = floor(log2 M)
     const int b = bitlen - 1;
     c.mp_precision = b / 2 - 1;

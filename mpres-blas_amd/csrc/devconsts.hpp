@@ -39,6 +39,11 @@ struct DevConsts {
     int h[P2T][MAXN];      // M_i mod 2^(j+1)
     int pow2inv[P2T][MAXN];// 2^-(j+1) mod m_i
     int mrcinv[MAXN][MAXN];// m_i^-1 mod m_j (j > i)
+    // positional form (pos.hpp), 16-bit limbs as doubles, least significant first
+    double pinv, pmod;               // 1 / M and M, rounded
+    double mi16[2 * MAXN][MAXN];     // limb l of M / m_i
+    double m16[2 * MAXN];            // limb l of M
+    double q16[2 * MAXN][MAXN];      // 2^(16 l) mod m_i
     const int *pow2;       // device pointer: RNS_POW2, (log2m + 1) x n, row-major
 };
 

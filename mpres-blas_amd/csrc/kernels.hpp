@@ -17,8 +17,9 @@
 // kernel (FULL = true, FIX = true) recomputes exactly the marked chains with
 // every case of the reference arithmetic. Both kernels run the identical
 // sequence of operations, so the result does not depend on which one
-// finished a chain. Over 8 moduli rounding is the common case and the
-// single full kernel is used.
+// finished a chain. Over 8 moduli rounding is the common case: the main
+// kernels there are the positional ones (kernels_pos.hpp), and the single full kernel
+// for the short chains of a dot.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -580,79 +581,6 @@ __global__ __launch_bounds__(BLK) void k_gemv_fold(const DevConsts *__restrict__
     else if (g.lane() == 0)
         *part.sign(v) = REDO;
 }
-// Residues of a run of `rows` consecutive elements of an SoA array (rows * N ints,
-// 16-byte aligned) moved to LDS with element stride N + 1. When a full run
-// (rows == W) is a whole number of 16-byte loads per thread (VEC), it goes
-// through registers in two halves, so that the next step's loads can be issued
-// before the current step computes: fetch issues the loads, store writes them
-// to LDS. Other runs are copied directly by store.
-// T: threads of the workgroup (BLK unless the kernel launches fewer).
-template <int N, int L, int T = BLK>
-struct RunStage {
-    static constexpr int W = T / L, SP = N + 1;
-    static constexpr bool VEC = (W * N) % (4 * T) == 0;
-    static constexpr int V4 = VEC ? W * N / 4 / T : 1;  // int4 per thread for a full run
-    int4 v[V4];
-    __device__ __forceinline__ void fetch(const int *src, int rows) {
-        if (VEC && rows == W) {
-            const int4 *s4 = (const int4 *)src;
-#pragma unroll
-            for (int q = 0; q < V4; q++) v[q] = s4[q * T + threadIdx.x];
-        }
-    }
-    __device__ __forceinline__ void store(int *sd, const int *src, int rows) const {
-        if (VEC && rows == W) {
-#pragma unroll
-            for (int q = 0; q < V4; q++) {
-                const int i = 4 * (q * T + threadIdx.x), e = i / N, f = i % N;
-                int *d = sd + e * SP + f;
-                d[0] = v[q].x;
-                d[1] = v[q].y;
-                d[2] = v[q].z;
-                d[3] = v[q].w;
-            }
-        } else {
-            for (int q = threadIdx.x; q < rows * N; q += T) sd[(q / N) * SP + q % N] = src[q];
-        }
-    }
-};
-
-// Main pass without transpose, the residues of A staged through LDS: workgroup
-// (x, t) holds the W = BLK / L consecutive rows o of block x, all with strided
-// index t, so each step j reads one contiguous run of column j of A. The run's
-// residues are loaded cooperatively (coalesced) into LDS with a padded stride and
-// every group reads its own from there. Same partials as k_gemv_fold.
-template <int N, int L, bool FULL>
-__global__ __launch_bounds__(BLK) void k_gemv_rows(const DevConsts *__restrict__ C, int m, int n, SoA A, int lda,
-                                                   AoSRef<N> bx, int b3, AoSRef<N> part) {
-    constexpr int W = BLK / L, R = N / L, SP = N + 1;
-    __shared__ int sd[W * SP];
-    A = rd(A);
-    const int gl = threadIdx.x / L;
-    const int t = blockIdx.y;
-    const long long o0 = (long long)blockIdx.x * W, o = o0 + gl;
-    const int rows = (int)((m - o0) < W ? (m - o0) : W);
-    bool ok = o < m;
-    Grp<N, L> g(C);
-    MP<R> acc;
-    g.zero(acc);
-    RunStage<N, L> stg;
-    if (t < n) stg.fetch(A.d + (o0 + (long long)t * lda) * N, rows);
-    for (int j = t; j < n; j += b3) {
-        stg.store(sd, A.d + (o0 + (long long)j * lda) * N, rows);
-        __syncthreads();
-        if (j + b3 < n) stg.fetch(A.d + (o0 + (long long)(j + b3) * lda) * N, rows);
-        if (ok) ok = g.template fma_step_d<FULL>(acc, A, o + (long long)j * lda, sd + gl * SP + g.lane() * R, bx, j);
-        __syncthreads();
-    }
-    if (o >= m) return;
-    const long long v = o * b3 + t;
-    if (ok)
-        store_aos(g, acc, part, v);
-    else if (g.lane() == 0)
-        *part.sign(v) = REDO;
-}
-
 // y[o] = y[o] (+) rowsum[o]  (src/blas/gemv.cuh:72-75 with mp_add rounding, add.cuh:223-248)
 template <int N, int L>
 __global__ __launch_bounds__(BLK) void k_gemv_final(const DevConsts *__restrict__ C, int len, SoA y, int incy,

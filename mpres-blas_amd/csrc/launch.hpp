@@ -81,18 +81,17 @@ struct Launch {
         }
         return hipGetLastError();
     }
-    // pass 0: the main kernel; pass 1: the fixup kernel over the chains the main
-    // kernel marked (16 and 32 moduli; nothing to do over 8 moduli)
+    // pass 0: the main kernel; pass 1: the fixup kernel over the chains marked
     static constexpr bool SPLIT = !Grp<N, L>::INL;
     template <int MODE>
     static void fold_pass(int pass, const dim3 &gr, const DevConsts *c, long long cnt, long long nvt, SoA xs, int incx,
                           SoA ys, int incy, AoSRef<N> XA, AoSRef<N> YA, AoSRef<N> O, hipStream_t st) {
         const dim3 bl(BLK);
-        if (pass == 0)
-            hipLaunchKernelGGL((k_fold<N, L, MODE, !SPLIT, false>), gr, bl, 0, st, c, cnt, nvt, xs, incx, ys, incy, XA,
-                               YA, O);
-        else if constexpr (SPLIT)
+        if (pass == 1)
             hipLaunchKernelGGL((k_fold<N, L, MODE, true, true>), gr, bl, 0, st, c, cnt, nvt, xs, incx, ys, incy, XA,
+                               YA, O);
+        else
+            hipLaunchKernelGGL((k_fold<N, L, MODE, !SPLIT, false>), gr, bl, 0, st, c, cnt, nvt, xs, incx, ys, incy, XA,
                                YA, O);
     }
     static hipError_t fold(const DevConsts *c, int mode, int pass, long long cnt, long long nvt, SoA xs, int incx,
@@ -169,8 +168,8 @@ struct Launch {
     // gemv passes: 0 preparation (split form: row minima of A's exponents, minimum
     // and pre-scaled residues of bx), 1 main kernel (split form: the residues), 2 split
     // form: the scalar chains (independent of pass 1, so a caller may run the two on two
-    // streams), 3 split form: the residues moved to the chains' results, then the fixup of
-    // marked partials. aux: the split form's bxp (N*n ints), EA (m ints), EB (1 int).
+    // streams), 3 split form: the residues moved to the chains' results, 4 the fixup of the
+    // partials still marked. Over 8 moduli the main kernel is the positional one (PosOps). aux: the split form's bxp (N*n ints), EA (m ints), EB (1 int).
     static bool gemv_split(bool trans, int b3) { return SPLIT && !trans && b3 <= 65535; }
     static size_t gemv_aux(bool trans, int m, int n) {
         return (SPLIT && !trans) ? 4 * ((size_t)N * n + m + 1) : 0;
@@ -198,12 +197,9 @@ struct Launch {
                 hipLaunchKernelGGL((k_gemv_resid<N, L>), dim3((m + RW - 1) / RW, b3), dim3(GV_RT), 0, st, c, m, n, A,
                                    lda, bxp, EA, EB, b3, part);
             }
-            else if (!TR && b3 <= 65535)  // grid y limit
-                hipLaunchKernelGGL((k_gemv_rows<N, L, !SPLIT>), dim3((m + BLK / L - 1) / (BLK / L), b3), bl, 0, st, c,
-                                   m, n, A, lda, bx, b3, part);
-            else
-                hipLaunchKernelGGL((k_gemv_fold<N, L, TR, !SPLIT, false>), gr, bl, 0, st, c, m, n, A, lda, bx, b3,
-                                   nvt, part);
+            else if constexpr (SPLIT)
+                hipLaunchKernelGGL((k_gemv_fold<N, L, TR, false, false>), gr, bl, 0, st, c, m, n, A, lda, bx, b3, nvt,
+                                   part);
         } else if (pass == 2) {
             if (split) {
                 const dim3 gc(grid_for((long long)m * b3, 1));
@@ -216,10 +212,11 @@ struct Launch {
                     hipLaunchKernelGGL((k_gemv_chain<N, L, false, false>), gc, bl, 0, st, c, m, n, A, lda, bx, b3,
                                        part);
             }
-        } else if constexpr (SPLIT) {
+        } else if (pass == 3) {
             if (split)
                 hipLaunchKernelGGL((k_gemv_scale<N, L>), dim3(grid_for(nvt * (N / GR), 1)), bl, 0, st, c, nvt, b3,
                                    (const int *)EA, (const int *)EB, part);
+        } else {
             hipLaunchKernelGGL((k_gemv_fold<N, L, TR, true, true>), gr, bl, 0, st, c, m, n, A, lda, bx, b3, nvt, part);
         }
     }
@@ -241,7 +238,7 @@ struct Launch {
     // gemm passes. Over 16 and 32 moduli (split form, see kernels.hpp):
     //   0 exponent minima and the int8 limb planes of the pre-scaled residues, 1 scalar chains,
     //   2 residue products (INT8 MFMA) and digits, 3 fixup of the marked chains, 4 epilogue.
-    // Over 8 moduli: 1 full sums, 4 epilogue. bits: bit length of the largest modulus.
+    // Over 8 moduli the sums are the positional kernel's (PosOps): 3 fixup, 4 epilogue. bits: bit length of the largest modulus.
     // ws: m*n sums, then (split form) the residue sums S (N*m*n ints), the minima (m + n
     // ints) and the limb planes of op(A) and op(B).
     static constexpr int GEMM_NL = 5;  // limbs per residue reserved (moduli below 2^35)
@@ -257,8 +254,7 @@ struct Launch {
     // Passes of the split-form gemm: 0 = exponent minima, int8 limb planes and the INT8 MFMA
     // residue products; 1 = the scalar chains; 2 = digits from both (needs 0 and 1); 3 = the
     // fixup of REDO chains; 4 = the alpha/beta epilogue. Passes 0 and 1 are independent, so a
-    // caller may run pass 0 on another stream. Over 8 moduli only pass 1 (the lane-group
-    // reduction) and pass 4 do work.
+    // caller may run pass 0 on another stream. Over 8 moduli only passes 3 and 4 do work.
     template <class VM>
     static void gemm_pass(int pass, const DevConsts *c, int bits, int ta, int tb, int m, int n, int k, VM A, int lda,
                           VM B, int ldb, char *ws, hipStream_t st) {
@@ -305,14 +301,11 @@ struct Launch {
                                    lda, B, ldb, sums);
             } else if (pass == 2) {
                 hipLaunchKernelGGL((k_gemm_digits<N, L>), dim3(grid_for(mn, 1)), bl, 0, st, c, m, n, S, EA, EB, sums);
-            } else if (pass == 3) {
-                hipLaunchKernelGGL((k_gemm_sum<N, L, true, true, VM>), gr, bl, 0, st, c, ta, tb, m, n, k, A, lda, B,
-                                   ldb, sums);
             }
-        } else if (pass == 1) {
-            hipLaunchKernelGGL((k_gemm_sum<N, L, true, false, VM>), gr, bl, 0, st, c, ta, tb, m, n, k, A, lda, B, ldb,
-                               sums);
         }
+        if (pass == 3)
+            hipLaunchKernelGGL((k_gemm_sum<N, L, true, true, VM>), gr, bl, 0, st, c, ta, tb, m, n, k, A, lda, B, ldb,
+                               sums);
     }
     static hipError_t gemm(const DevConsts *c, int pass, int bits, int m, int n, int k, SoA alpha, SoA A, int lda,
                            SoA B, int ldb, SoA beta, SoA Cm, int ldc, char *ws, hipStream_t st) {

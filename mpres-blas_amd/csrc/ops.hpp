@@ -65,7 +65,8 @@ struct Ops {
     // comparisons (mode 0 mp_cmp, 1 mp_cmp_abs on AoS numbers, 2 rns_cmp on bare residues)
     hipError_t (*cmp)(const DevConsts *, int, int, const char *, const char *, const int *, const int *, int *,
                       hipStream_t);
-    // the reduction launchers take a pass: 0 = main kernel, 1 = fixup kernel (see kernels.hpp);
+    // the reduction launchers take a pass: 0 = main kernel (over 8 moduli only the short chains of dot: the
+    // others are PosOps'), 1 = fixup kernel (see kernels.hpp);
     // gemv_fold runs passes 0..3 and gemm / gemm_v2 passes 0..4 (see launch.hpp)
     hipError_t (*fold)(const DevConsts *, int, int, long long, long long, SoA, int, SoA, int, const char *,
                        const char *, char *, hipStream_t);
@@ -110,6 +111,24 @@ struct Ops {
     // batched form: reset the work queue, then the persistent kernel over `count` items on `grid` workgroups
     hipError_t (*batch)(const DevConsts *, const BatchItem *, int, int *, char *, int, hipStream_t);
 };
+
+// The reduction chains on positional integers (kernels_pos.hpp), over 8 moduli. What they cannot do
+// they mark REDO for the residue kernels' fixup pass.
+struct PosOps {
+    hipError_t (*fold)(const DevConsts *, int, long long, long long, SoA, int, SoA, int, const char *, const char *,
+                       char *, hipStream_t);
+    size_t (*rec_bytes)(long long);
+    // records of op(A) (side 0, cnt rows) or op(B) (side 1, cnt columns), k terms
+    hipError_t (*records)(const DevConsts *, int, int, int, int, SoA, const char *, bool, int, char *, hipStream_t);
+    hipError_t (*gemv)(const DevConsts *, bool, int, int, SoA, int, const char *, const char *, int, long long, char *,
+                       hipStream_t);
+    hipError_t (*gemm)(const DevConsts *, int, int, int, int, int, SoA, int, SoA, int, const char *, const char *,
+                       char *, hipStream_t);
+    hipError_t (*gemm_v2)(const DevConsts *, int, int, int, int, int, const char *, int, const char *, int,
+                          const char *, const char *, char *, hipStream_t);
+};
+const PosOps *pos_ops_n8();
+inline const PosOps *pos_ops(int n) { return n == 8 ? pos_ops_n8() : nullptr; }
 
 // Compiled (moduli count, lanes per number) variants; each has its own
 // translation unit csrc/k_n<N>_l<L>.hip defining ops_n<N>_l<L>().

@@ -990,15 +990,17 @@ int mpres_gemv(mpres_ctx_t *c, int trans, int m, int n, const mp_array_t *alpha,
 
 // ---------------------------------------------------------------- gemm
 // the m*n dot-product sums, and over 16/32 moduli the pre-scaled residue planes; after them
-// (mpres_gemm_workspace) the positional kernel's records of A and B, which a smaller workspace
-// goes without
+// (mpres_gemm_workspace) what a smaller workspace goes without: over 8 moduli the positional
+// kernel's records of A and B, over 16 and 32 the scalar chains' operands
 static size_t gemm_need(const mpres_ctx_t *c, int m, int n, int k) { return c->ops[OP_GEMM]->gemm_ws(m, n, k); }
 static size_t gemm_rec_bytes(const mpres_ctx_t *c, int cnt, int k) {
     return (c->pos->rec_bytes((long long)cnt * k) + 255) / 256 * 256;
 }
 size_t mpres_gemm_workspace(const mpres_ctx_t *c, int m, int n, int k) {
     if (!c || m <= 0 || n <= 0 || k < 0) return 0;
-    return gemm_need(c, m, n, k) + (c->pos ? 256 + gemm_rec_bytes(c, m, k) + gemm_rec_bytes(c, n, k) : 0);
+    const size_t more = c->pos ? gemm_rec_bytes(c, m, k) + gemm_rec_bytes(c, n, k)
+                               : c->ops[OP_GEMM]->gemm_chain_ws(m, n, k);
+    return gemm_need(c, m, n, k) + (more ? more + 256 : 0);
 }
 
 int mpres_gemm(mpres_ctx_t *c, int ta, int tb, int m, int n, int k, const mp_array_t *alpha, const mp_array_t *A,
@@ -1020,7 +1022,8 @@ int mpres_gemm(mpres_ctx_t *c, int ta, int tb, int m, int n, int k, const mp_arr
     const size_t need = gemm_need(c, m, n, k);
     int rc = wu.get2(ws, wsb, need, mpres_gemm_workspace(c, m, n, k), &w, &full);
     if (rc) return rc;
-    char *ra = full ? w + (need + 255) / 256 * 256 : nullptr, *rb = full ? ra + gemm_rec_bytes(c, m, k) : nullptr;
+    char *ra = full ? w + (need + 255) / 256 * 256 : nullptr;
+    char *rb = full && c->pos ? ra + gemm_rec_bytes(c, m, k) : nullptr;
     const Ops *o = sized(c, OP_GEMM, (long long)m * n * k);
     if (c->host.n == 8) {
         if (full) {
@@ -1033,7 +1036,7 @@ int mpres_gemm(mpres_ctx_t *c, int ta, int tb, int m, int n, int k, const mp_arr
         }
         for (int pass = 3; pass < 5; pass++)
             HIPCHK(o->gemm(c->dev, pass, c->bits, m, n, k, soa_of(alpha), soa_of(A), lda, soa_of(B), ldb, soa_of(beta),
-                           soa_of(C), ldc, w, strm(st)));
+                           soa_of(C), ldc, w, ra, strm(st)));
         return MPRES_OK;
     }
     // the residue path (pass 0) runs on the side stream while the chains (pass 1) run on st
@@ -1041,17 +1044,17 @@ int mpres_gemm(mpres_ctx_t *c, int ta, int tb, int m, int n, int k, const mp_arr
     {
         ProfScope ps(c, PROF_GEMM_RESID, fk.s1);
         HIPCHK(o->gemm(c->dev, 0, c->bits, m, n, k, soa_of(alpha), soa_of(A), lda, soa_of(B), ldb, soa_of(beta),
-                       soa_of(C), ldc, w, fk.s1));
+                       soa_of(C), ldc, w, ra, fk.s1));
     }
     {
         ProfScope ps(c, OP_GEMM, strm(st));
         HIPCHK(o->gemm(c->dev, 1, c->bits, m, n, k, soa_of(alpha), soa_of(A), lda, soa_of(B), ldb, soa_of(beta),
-                       soa_of(C), ldc, w, strm(st)));
+                       soa_of(C), ldc, w, ra, strm(st)));
     }
     HIPCHK(fk.join());
     for (int pass = 2; pass < 5; pass++)
         HIPCHK(o->gemm(c->dev, pass, c->bits, m, n, k, soa_of(alpha), soa_of(A), lda, soa_of(B), ldb, soa_of(beta),
-                       soa_of(C), ldc, w, strm(st)));
+                       soa_of(C), ldc, w, ra, strm(st)));
     return MPRES_OK;
 }
 
@@ -1092,12 +1095,13 @@ int mpres_gemm_v2(mpres_ctx_t *c, int ta, int tb, int m, int n, int k, const voi
     const size_t need = gemm_need(c, m, n, k);
     int rc = wu.get2(ws, wsb, need, mpres_gemm_workspace(c, m, n, k), &w, &full);
     if (rc) return rc;
-    char *ra = full ? w + (need + 255) / 256 * 256 : nullptr, *rb = full ? ra + gemm_rec_bytes(c, m, k) : nullptr;
+    char *ra = full ? w + (need + 255) / 256 * 256 : nullptr;
+    char *rb = full && c->pos ? ra + gemm_rec_bytes(c, m, k) : nullptr;
     const int tra = ta == MPRES_TRANS || ta == MPRES_CONJ_TRANS, trb = tb == MPRES_TRANS || tb == MPRES_CONJ_TRANS;
     // as in mpres_gemm: the residue path (pass 0) on the side stream, the chains on st
     const Ops *o = sized(c, OP_GEMM, (long long)m * n * k);
     Fork fk(c, strm(st));
-    if (full) {
+    if (full && c->pos) {
         HIPCHK(c->pos->records(c->dev, 0, tra, m, k, SoA{}, (const char *)A, false, lda, ra, fk.s1));
         HIPCHK(c->pos->records(c->dev, 1, trb, n, k, SoA{}, (const char *)B, false, ldb, rb, fk.s1));
     }
@@ -1107,7 +1111,7 @@ int mpres_gemm_v2(mpres_ctx_t *c, int ta, int tb, int m, int n, int k, const voi
             HIPCHK(c->pos->gemm_v2(c->dev, tra, trb, m, n, k, (const char *)A, lda, (const char *)B, ldb, ra, rb, w,
                                    strm(st)));
         HIPCHK(o->gemm_v2(c->dev, pass, c->bits, tra, trb, m, n, k, (const char *)alpha, (const char *)A,
-                                        lda, (const char *)B, ldb, (const char *)beta, (char *)C, ldc, w,
+                                        lda, (const char *)B, ldb, (const char *)beta, (char *)C, ldc, w, ra,
                                         pass == 0 ? fk.s1 : strm(st)));
     }
     return MPRES_OK;

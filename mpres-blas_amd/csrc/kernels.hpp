@@ -833,18 +833,12 @@ __global__ __launch_bounds__(BLK) void k_gemm_limbs(const DevConsts *__restrict_
             P[((size_t)r * nl + a) * plane + pos] = (signed char)((v >> (LIMB_BITS * a)) & ((1 << LIMB_BITS) - 1));
     }
 }
-// scalar chain of every entry (one thread per entry): the sum's sign, exponent and
-// interval evaluation into the workspace, or REDO
-template <int N, int L, class VM>
-__global__ __launch_bounds__(BLK) void k_gemm_chain(const DevConsts *__restrict__ C, int ta, int tb, int m, int n,
-                                                    int k, VM A, int lda, VM B, int ldb, AoSRef<N> sums) {
-    if constexpr (std::is_same<VM, SoA>::value) {
-        A = rd(A);
-        B = rd(B);
-    }
-    const long long e = (long long)blockIdx.x * BLK + threadIdx.x;
-    if (e >= (long long)m * n) return;
-    const int row = (int)(e % m), col = (int)(e / m);
+// scalar chain of one entry by sc_fma_step: the sum's sign, exponent and interval evaluation into
+// the workspace, or REDO
+template <int N, class VM>
+__device__ __forceinline__ void gemm_chain_entry(const DevConsts *__restrict__ C, int ta, int tb, int k, const VM &A,
+                                                 int lda, const VM &B, int ldb, int row, int col, AoSRef<N> sums,
+                                                 long long e) {
     const ScC K = sc_consts(C);
     Sc acc{0, 0, Er{0.0, 0}, Er{0.0, 0}};
     bool ok = true;
@@ -865,6 +859,188 @@ __global__ __launch_bounds__(BLK) void k_gemm_chain(const DevConsts *__restrict_
     ErMem *ev = sums.eval(e);
     ev[0] = ErMem{acc.ev0.frac, (long long)acc.ev0.exp};
     ev[1] = ErMem{acc.ev1.frac, (long long)acc.ev1.exp};
+}
+// scalar chain of every entry (one thread per entry)
+template <int N, int L, class VM>
+__global__ __launch_bounds__(BLK) void k_gemm_chain(const DevConsts *__restrict__ C, int ta, int tb, int m, int n,
+                                                    int k, VM A, int lda, VM B, int ldb, AoSRef<N> sums) {
+    if constexpr (std::is_same<VM, SoA>::value) {
+        A = rd(A);
+        B = rd(B);
+    }
+    const long long e = (long long)blockIdx.x * BLK + threadIdx.x;
+    if (e >= (long long)m * n) return;
+    gemm_chain_entry<N>(C, ta, tb, k, A, lda, B, ldb, (int)(e % m), (int)(e / m), sums, e);
+}
+
+// ---- scalar chains on absolute bounds ----
+// A chain's interval bounds as plain doubles: lower and upper bound of the value itself (the
+// evaluation times 2^exp, scaled by 2^(log2 M)) instead of fractions with exponents beside them.
+// Scaling by powers of two is exact and commutes with directed rounding as long as nothing
+// leaves the double range, so for operands of ordinary size (bounds within 2^-CA_RANGE ..
+// 2^CA_RANGE) each step rounds exactly as sc_fma_step does, and what remains of a step is
+// the twelve directed operations and a few integer ones (33 vector instructions instead of
+// 161; 512^3 at 32 moduli 820 -> 199 us, 300^3 at 16 moduli 294 -> 97 us, issue-bound). The exact-step conditions move to the end of the chain: no step rounded or dropped an
+// operand if the sum of all |product| bounds, at the smallest exponent, stays below the
+// rounding threshold. Chains that this does not show (or that end in a zero bound, or hold an
+// operand of unusual size) run sc_fma_step.
+constexpr int CA_RANGE = 200;  // sums of products stay within 2^+-500: no exponent difference leaves the double range
+struct ChainOp {
+    double lo, hi;  // bounds of |value|; lo carries the number's sign bit
+};
+// exponent of an operand outside the range (the smallest sums mark the chain)
+constexpr int CA_BAD = -(1 << 24);
+// bounds and exponents of op(A) (m x k, rows fastest; blockIdx.y = 0) and op(B) (k x n, k fastest; 1)
+template <int N, int SIDE, class VM>
+__device__ __forceinline__ void chain_ops_at(const DevConsts *__restrict__ C, long long g, int cnt, int k, int t,
+                                             const VM &X, int ld, ChainOp *__restrict__ ops, int *__restrict__ ex) {
+    if (g >= (long long)cnt * k) return;
+    const int j = SIDE == 0 ? (int)(g % cnt) : (int)(g / k), i = SIDE == 0 ? (int)(g / cnt) : (int)(g % k);
+    int s, e;
+    Er e0, e1;
+    scalars_of<N>(X, op_index<SIDE>(t, j, i, ld), s, e, e0, e1);
+    const int L = C->log2m, a0 = e0.exp + e + L, a1 = e1.exp + e + L;
+    const bool zero = e0.frac == 0 && e1.frac == 0;
+    const bool fits = zero || (e0.frac > 0 && a0 >= -CA_RANGE && a0 <= CA_RANGE && a1 >= -CA_RANGE && a1 <= CA_RANGE);
+    const double lo = fits ? ldexp(e0.frac, a0) : 0.0;
+    ops[g] = ChainOp{s ? -lo : lo, fits ? ldexp(e1.frac, a1) : 0.0};
+    ex[g] = fits ? e : CA_BAD;
+}
+template <int N, class VM>
+__global__ __launch_bounds__(BLK) void k_chain_ops(const DevConsts *__restrict__ C, int ta, int tb, int m, int n, int k,
+                                                   VM A, int lda, VM B, int ldb, ChainOp *__restrict__ pa,
+                                                   int *__restrict__ ea, ChainOp *__restrict__ pb,
+                                                   int *__restrict__ eb) {
+    const long long g = (long long)blockIdx.x * BLK + threadIdx.x;
+    if (blockIdx.y == 0) {
+        if constexpr (std::is_same<VM, SoA>::value) A = rd(A);
+        chain_ops_at<N, 0>(C, g, m, k, ta, A, lda, pa, ea);
+    } else {
+        if constexpr (std::is_same<VM, SoA>::value) B = rd(B);
+        chain_ops_at<N, 1>(C, g, n, k, tb, B, ldb, pb, eb);
+    }
+}
+// One step under round-down (chain_rd): lo += the product's lower bound, hn += minus its upper
+// bound (upper bounds are kept negated, so that one rounding mode serves both), mag += minus its
+// magnitude. The quotient by the evaluation unit: q = x (zh + zl) rounded down, where zh + zl
+// exceeds 1/z by 2^-102 relative for the lower bound and falls short of it for the (negated)
+// upper one, is the rounded-down quotient or its upper neighbour; the exact remainder's sign
+// then decides (divk_rd).
+struct ChainK {
+    double uf, uh, ul, lf, lh, ll;  // unit_upp and unit_low: fraction, two-double reciprocals biased as above
+};
+__device__ __forceinline__ ChainK chain_consts(const DevConsts *C) {
+    const ScC K = sc_consts(C);
+    return ChainK{K.uuf, K.uu_rh, fma(K.uu_rh, 0x1p-102, K.uu_rl), K.ulf, K.ul_rh, fma(K.ul_rh, -0x1p-102, K.ul_rl)};
+}
+__device__ __forceinline__ void chain_rd(bool on) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if (on)
+        asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 2\n\ts_nop 1");
+    else
+        asm volatile("s_nop 1\n\ts_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 0\n\ts_nop 1");
+#else
+    (void)on;
+#endif
+}
+__device__ __forceinline__ void chain_step(const ChainK &K, const ChainOp &x, const ChainOp &y, double &lo, double &hn,
+                                           double &mag) {
+    double p, n;  // the product's lower bound, and minus its upper bound
+#if defined(__HIP_DEVICE_COMPILE__)
+    double a, b, t, u;
+    asm volatile("v_mul_f64 %0, |%1|, |%2|" : "=v"(a) : "v"(x.lo), "v"(y.lo));
+    asm volatile("v_mul_f64 %0, -%1, %2" : "=v"(b) : "v"(x.hi), "v"(y.hi));
+    asm volatile("v_mul_f64 %0, %1, %2" : "=v"(t) : "v"(a), "s"(K.ul));
+    asm volatile("v_mul_f64 %0, %1, %2" : "=v"(u) : "v"(b), "s"(K.ll));
+    asm volatile("v_fma_f64 %0, %1, %2, %3" : "=v"(p) : "v"(a), "s"(K.uh), "v"(t));
+    asm volatile("v_fma_f64 %0, %1, %2, %3" : "=v"(n) : "v"(b), "s"(K.lh), "v"(u));
+    asm volatile("v_fma_f64 %0, -%1, %2, %3" : "=v"(a) : "v"(p), "s"(K.uf), "v"(a));
+    asm volatile("v_fma_f64 %0, -%1, %2, %3" : "=v"(b) : "v"(n), "s"(K.lf), "v"(b));
+    asm volatile("v_fma_f64 %0, %1, %2, %3" : "=v"(p) : "v"(a), "s"(0x1p-64), "v"(p));
+    asm volatile("v_fma_f64 %0, %1, %2, %3" : "=v"(n) : "v"(b), "s"(0x1p-64), "v"(n));
+    const bool neg = (int)((uint32_t)(d2u(x.lo) >> 32) ^ (uint32_t)(d2u(y.lo) >> 32)) < 0;
+    const double pl = neg ? n : p, ph = neg ? p : n;
+    asm volatile("v_add_f64 %0, %1, %2" : "=v"(lo) : "v"(lo), "v"(pl));
+    asm volatile("v_add_f64 %0, %1, %2" : "=v"(hn) : "v"(hn), "v"(ph));
+    asm volatile("v_add_f64 %0, %1, %2" : "=v"(mag) : "v"(mag), "v"(n));
+#else
+    const double a = mul_rd(fabs(x.lo), fabs(y.lo)), b = mul_ru(x.hi, y.hi);
+    p = a == 0 ? a : div_rd(a, K.uf);
+    n = b == 0 ? b : -div_ru(b, K.lf);
+    const bool neg = (d2u(x.lo) ^ d2u(y.lo)) >> 63;
+    lo = add_rd(lo, neg ? n : p);
+    hn = add_rd(hn, neg ? p : n);
+    mag = add_rd(mag, n);
+#endif
+}
+// Scalar chain of every entry on the operands of k_chain_ops (A: record row + m i, B: i + k col);
+// results as k_gemm_chain. One thread per entry; the operands of step i + 1 are loaded before
+// step i runs.
+// UB: m is a multiple of 64, so a wave's entries share a column and read its operands once.
+template <int N, bool UB, class VM>
+__global__ __launch_bounds__(BLK) void k_gemm_chain_abs(const DevConsts *__restrict__ C, int ta, int tb, int m, int n,
+                                                        int k, VM A, int lda, VM B, int ldb,
+                                                        const ChainOp *__restrict__ pa, const int *__restrict__ ea,
+                                                        const ChainOp *__restrict__ pb, const int *__restrict__ eb,
+                                                        AoSRef<N> sums) {
+    const long long e = (long long)blockIdx.x * BLK + threadIdx.x;
+    if (e >= (long long)m * n) return;
+    const int row = (int)(e % m);
+    int col = (int)(e / m);
+    if constexpr (UB) col = __builtin_amdgcn_readfirstlane(col);
+    const long long b0 = (long long)col * k;
+    const ChainK K = chain_consts(C);
+    double lo = 0, hn = 0, mag = 0;
+    int E = 0;
+    bool straddle = false;
+    if (k > 0) {
+        const ChainOp *px = pa + row, *py = pb + b0;
+        const int *qx = ea + row, *qy = eb + b0;
+        ChainOp x = *px, y = *py;
+        int pe = *qx + *qy;
+        auto step = [&] {
+            E = pe < E ? pe : E;
+            chain_step(K, x, y, lo, hn, mag);
+            straddle = straddle || ((lo < 0) != (hn > 0));
+        };
+        chain_rd(true);
+        for (int i = 1; i < k; i++) {
+            px += m;
+            qx += m;
+            const ChainOp nx = *px, ny = py[i];
+            const int npe = *qx + qy[i];
+            step();
+            x = nx;
+            y = ny;
+            pe = npe;
+        }
+        step();
+        chain_rd(false);
+    }
+    // scale of the bounds: the evaluation's is 2^-(2 log2 M + unit exponent) smaller
+    const int sl = 2 * C->log2m + C->unit_upp.exp, su = 2 * C->log2m + C->unit_low.exp;
+    const double top = -mag;
+    const bool sure = lo != 0 && hn != 0 && E > CA_BAD / 2 && sl == su &&
+                      er_set_d(top).exp + 2 - sl - E < C->mp_h;  // no step rounded or dropped an operand
+    if (!sure) {
+        if constexpr (std::is_same<VM, SoA>::value) {
+            A = rd(A);
+            B = rd(B);
+        }
+        gemm_chain_entry<N>(C, ta, tb, k, A, lda, B, ldb, row, col, sums, e);
+        return;
+    }
+    if (straddle) {
+        *sums.sign(e) = REDO;
+        return;
+    }
+    const int sign = lo < 0;
+    const Er f0 = er_adjust(sign ? hn : lo, -sl - E), f1 = er_adjust(sign ? -lo : -hn, -sl - E);
+    *sums.sign(e) = sign;
+    *sums.exp(e) = E;
+    ErMem *ev = sums.eval(e);
+    ev[0] = ErMem{f0.frac, (long long)f0.exp};
+    ev[1] = ErMem{f1.frac, (long long)f1.exp};
 }
 
 // k_gemm_chain for the v1 layout and op(A) = A, op(B) = B, with every element offset of A

@@ -255,9 +255,16 @@ struct Launch {
     // residue products; 1 = the scalar chains; 2 = digits from both (needs 0 and 1); 3 = the
     // fixup of REDO chains; 4 = the alpha/beta epilogue. Passes 0 and 1 are independent, so a
     // caller may run pass 0 on another stream. Over 8 moduli only passes 3 and 4 do work.
+    // bytes of the scalar chains' operands (k_chain_ops)
+    static size_t gemm_chain_ws(int m, int n, int k) {
+        return SPLIT && k >= CHAIN_OPS_K ? (sizeof(ChainOp) + 4) * ((size_t)m + n) * k + 16 : 0;
+    }
+    // k from which the chains read prepared operands (k_gemm_chain_abs): preparing them costs a
+    // launch (about 5 us), a step of the chain 0.1 us instead of 0.5 us
+    static constexpr int CHAIN_OPS_K = 16;
     template <class VM>
     static void gemm_pass(int pass, const DevConsts *c, int bits, int ta, int tb, int m, int n, int k, VM A, int lda,
-                          VM B, int ldb, char *ws, hipStream_t st) {
+                          VM B, int ldb, char *ws, char *ops, hipStream_t st) {
         const long long mn = (long long)m * n;
         const dim3 gr(grid_for(mn, L)), bl(BLK);
         const AoSRef<N> sums{ws};
@@ -284,8 +291,22 @@ struct Launch {
                 hipLaunchKernelGGL((k_gemm_limbs<N, L, VM, 1>), dim3(grid_for((long long)NP * KP, 1)), bl, 0, st, c, n,
                                    NP, k, KP, nl, tb, B, ldb, EB, PB);
                 mf_products(c, nl, m, n, MP, NP, KP, PA, PB, nullptr, nullptr, S, st);
+            } else if (pass == 1 && ops) {
+                ChainOp *pa = (ChainOp *)(ops + (16 - (uintptr_t)ops % 16) % 16), *pb = pa + (size_t)m * k;
+                int *ea = (int *)(pb + (size_t)n * k), *eb = ea + (size_t)m * k;
+                const long long most = (long long)(m > n ? m : n) * k;
+                hipLaunchKernelGGL((k_chain_ops<N, VM>), dim3(grid_for(most, 1), 2), bl, 0, st, c, ta, tb, m, n, k, A,
+                                   lda, B, ldb, pa, ea, pb, eb);
+                if (m % 64 == 0)
+                    hipLaunchKernelGGL((k_gemm_chain_abs<N, true, VM>), dim3(grid_for(mn, 1)), bl, 0, st, c, ta, tb, m,
+                                       n, k, A, lda, B, ldb, (const ChainOp *)pa, (const int *)ea, (const ChainOp *)pb,
+                                       (const int *)eb, sums);
+                else
+                    hipLaunchKernelGGL((k_gemm_chain_abs<N, false, VM>), dim3(grid_for(mn, 1)), bl, 0, st, c, ta, tb,
+                                       m, n, k, A, lda, B, ldb, (const ChainOp *)pa, (const int *)ea,
+                                       (const ChainOp *)pb, (const int *)eb, sums);
             } else if (pass == 1) {
-                // no transposes and element offsets below 2^28: the specialised chain kernel
+                // a workspace without room for the operands, or short chains: no transposes and element offsets below 2^28: the specialised chain kernel
                 if constexpr (std::is_same<VM, SoA>::value) {
                     if (ta == 0 && tb == 0 && (long long)lda * k <= (1LL << 28) && (long long)ldb * n <= (1LL << 28)) {
                         if (m % 64 == 0)
@@ -308,10 +329,10 @@ struct Launch {
                                sums);
     }
     static hipError_t gemm(const DevConsts *c, int pass, int bits, int m, int n, int k, SoA alpha, SoA A, int lda,
-                           SoA B, int ldb, SoA beta, SoA Cm, int ldc, char *ws, hipStream_t st) {
+                           SoA B, int ldb, SoA beta, SoA Cm, int ldc, char *ws, char *ops, hipStream_t st) {
         if ((long long)m * n <= 0) return hipSuccess;
         if (pass < 4)
-            gemm_pass<SoA>(pass, c, bits, 0, 0, m, n, k, A, lda, B, ldb, ws, st);
+            gemm_pass<SoA>(pass, c, bits, 0, 0, m, n, k, A, lda, B, ldb, ws, ops, st);
         else
             hipLaunchKernelGGL((k_gemm_fin<N, L, false, SoA>), dim3(grid_for((long long)m * n, L)), dim3(BLK), 0, st,
                                c, m, n, alpha, beta, Cm, ldc, AoSRef<N>{ws});
@@ -319,11 +340,11 @@ struct Launch {
     }
     static hipError_t gemm_v2(const DevConsts *c, int pass, int bits, int ta, int tb, int m, int n, int k,
                               const char *alpha, const char *A, int lda, const char *B, int ldb, const char *beta,
-                              char *Cm, int ldc, char *ws, hipStream_t st) {
+                              char *Cm, int ldc, char *ws, char *ops, hipStream_t st) {
         if ((long long)m * n <= 0) return hipSuccess;
         if (pass < 4)
             gemm_pass<AoSRef<N>>(pass, c, bits, ta, tb, m, n, k, AoSRef<N>{(char *)A}, lda, AoSRef<N>{(char *)B}, ldb,
-                                 ws, st);
+                                 ws, ops, st);
         else
             hipLaunchKernelGGL((k_gemm_fin<N, L, true, AoSRef<N>>), dim3(grid_for((long long)m * n, L)), dim3(BLK),
                                0, st, c, m, n, AoSRef<N>{(char *)alpha}, AoSRef<N>{(char *)beta}, AoSRef<N>{Cm}, ldc,
@@ -611,6 +632,7 @@ struct Launch {
         o.gemv_final = &gemv_final;
         o.gemm = &gemm;
         o.gemm_ws = &gemm_ws;
+        o.gemm_chain_ws = &gemm_chain_ws;
         o.gemv_aux = &gemv_aux;
         o.gemm_mfma = &gemm_mfma;
         o.gemm_mfma_ws = &gemm_mfma_ws;

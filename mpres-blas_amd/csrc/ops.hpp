@@ -84,10 +84,11 @@ struct Ops {
     size_t (*gemv_aux)(bool, int, int);
     hipError_t (*gemv_final)(const DevConsts *, int, SoA, int, const char *, hipStream_t);
     hipError_t (*gemm)(const DevConsts *, int, int, int, int, int, SoA, SoA, int, SoA, int, SoA, SoA, int, char *,
-                       hipStream_t);
+                       char *, hipStream_t);
     hipError_t (*gemm_v2)(const DevConsts *, int, int, int, int, int, int, int, const char *, const char *, int,
-                          const char *, int, const char *, char *, int, char *, hipStream_t);
+                          const char *, int, const char *, char *, int, char *, char *, hipStream_t);
     size_t (*gemm_ws)(int, int, int);
+    size_t (*gemm_chain_ws)(int, int, int);
     hipError_t (*gemm_mfma)(const DevConsts *, int, int, int, int, int, int, int, SoA, SoA, int, SoA, int, SoA, SoA,
                             int, char *, hipStream_t);
     size_t (*gemm_mfma_ws)(int, int, int, int);

@@ -74,7 +74,11 @@ const Ops *find_ops(int n, int L) { return find_variant(n, L); }
 // logic); reductions with few independent chains prefer more lanes.
 // Lanes by call size measured on MI355X (mpres-blas_amd/lanes_tune.py, the table in
 // mpres-blas_amd/tuning/lanes_gfx950.json): a call of size <= bound[i] uses lanes[i], a
-// larger one the last entry. Installed at context creation for these sets; mpres_set_lanes
+// larger one the last entry. That table is of operands that are doubles; the axpy, element, gemm
+// and SpMV entries over 16 and 32 moduli weigh full operands, whose every product rounds, as
+// well: with one lane a number (two at 16 moduli up to 65536) they round positionally, axpy_v2 of
+// 120000 numbers of 212 bits 0.058 ms against 0.32 with 4 lanes (doubles 0.013 and 0.011), and
+// with one modulus a lane the rounding is inlined (20000 numbers 0.033 against 0.11 ms). Installed at context creation for these sets; mpres_set_lanes
 // replaces an operation's table by a fixed choice, mpres_set_lanes(op, 0) restores it.
 struct BuiltinLanes {
     const char *set;
@@ -90,17 +94,17 @@ const BuiltinLanes kBuiltinLanes[] = {
     {"8_2double", OP_SPMV, 3, {31622LL, 316227LL, 1000000LL}, {8, 8, 8}},
     {"8_2double", OP_ELEM, 3, {16384LL, 262144LL, 1048576LL}, {8, 2, 2}},
     {"16_4double", OP_DOT, 4, {16384LL, 262144LL, 4194304LL, 16777216LL}, {16, 16, 4, 4}},
-    {"16_4double", OP_AXPY, 4, {16384LL, 262144LL, 4194304LL, 16777216LL}, {16, 4, 1, 1}},
+    {"16_4double", OP_AXPY, 3, {24576LL, 65536LL, 16777216LL}, {16, 2, 1}},
     {"16_4double", OP_GEMV, 4, {16384LL, 262144LL, 4194304LL, 16777216LL}, {16, 16, 16, 16}},
-    {"16_4double", OP_GEMM, 4, {741455LL, 5931641LL, 47453132LL, 134217728LL}, {16, 16, 4, 4}},
-    {"16_4double", OP_SPMV, 3, {31622LL, 316227LL, 1000000LL}, {2, 4, 4}},
-    {"16_4double", OP_ELEM, 3, {16384LL, 262144LL, 1048576LL}, {16, 4, 4}},
+    {"16_4double", OP_GEMM, 1, {134217728LL}, {16}},
+    {"16_4double", OP_SPMV, 1, {1000000LL}, {16}},
+    {"16_4double", OP_ELEM, 2, {32768LL, 1048576LL}, {16, 1}},
     {"32_8double", OP_DOT, 4, {16384LL, 262144LL, 4194304LL, 16777216LL}, {32, 8, 8, 8}},
-    {"32_8double", OP_AXPY, 4, {16384LL, 262144LL, 4194304LL, 16777216LL}, {8, 8, 1, 1}},
+    {"32_8double", OP_AXPY, 2, {16384LL, 16777216LL}, {32, 1}},
     {"32_8double", OP_GEMV, 4, {16384LL, 262144LL, 4194304LL, 16777216LL}, {32, 4, 8, 8}},
     {"32_8double", OP_GEMM, 4, {741455LL, 5931641LL, 47453132LL, 134217728LL}, {8, 8, 8, 8}},
-    {"32_8double", OP_SPMV, 3, {31622LL, 316227LL, 1000000LL}, {1, 2, 4}},
-    {"32_8double", OP_ELEM, 3, {16384LL, 262144LL, 1048576LL}, {32, 8, 8}},
+    {"32_8double", OP_SPMV, 1, {1000000LL}, {32}},
+    {"32_8double", OP_ELEM, 2, {16384LL, 1048576LL}, {32, 1}},
 };
 
 int default_lanes(int n, int op) {
@@ -126,6 +130,7 @@ struct mpres_ctx {
     // entry i serves calls of size <= bound[i], the last entry larger ones
     struct LanesTable {
         int count = 0;
+        bool builtin = false;
         long long bound[MPRES_LANES_TABLE_MAX] = {};
         const Ops *ops[MPRES_LANES_TABLE_MAX] = {};
     } lt[OP_COUNT];
@@ -164,6 +169,7 @@ void install_builtin_lanes(mpres_ctx *c, int op) {
             if (!t.ops[i]) return;
         }
         t.count = b.count;
+        t.builtin = true;
         return;
     }
 }
@@ -416,7 +422,7 @@ static int table_of(const DevConsts &h, const std::vector<int> &pow2, int what, 
     switch (what) {
         case 0: put(h.m, n * sizeof(int)); break;
         case 1: put(h.w, n * sizeof(int)); break;
-        case 2: put(pow2.data(), pow2.size() * sizeof(int)); break;
+        case 2: put(pow2.data(), (size_t)(h.log2m + 1) * n * sizeof(int)); break;
         case 3: put(h.mpow2, sizeof h.mpow2); break;
         case 4:
             for (int j = 0; j < P2T; j++) put(h.h[j], n * sizeof(int));
@@ -570,7 +576,7 @@ int mpres_array_device2host(mpres_ctx_t *c, void *dst, const mp_array_t *src, si
 int mpres_array_set_d(mpres_ctx_t *c, mp_array_t *dst, const double *x, int count, void *st) {
     if (!c || !dst || (!x && count > 0)) return fail(MPRES_ERR_ARG, "null argument");
     if (count <= 0) return MPRES_OK;
-    HIPCHK(c->ops[OP_ELEM]->set_d(c->dev, x, count, soa_of(dst), nullptr, true, strm(st)));
+    HIPCHK(sized(c, OP_ELEM, count)->set_d(c->dev, x, count, soa_of(dst), nullptr, true, strm(st)));
     return MPRES_OK;
 }
 
@@ -578,7 +584,7 @@ int mpres_set_d(mpres_ctx_t *c, void *dst, const double *x, int count, void *st)
     if (!c || (!dst && count > 0) || (!x && count > 0)) return fail(MPRES_ERR_ARG, "null argument");
     if (count <= 0) return MPRES_OK;
     SoA none{};
-    HIPCHK(c->ops[OP_ELEM]->set_d(c->dev, x, count, none, (char *)dst, false, strm(st)));
+    HIPCHK(sized(c, OP_ELEM, count)->set_d(c->dev, x, count, none, (char *)dst, false, strm(st)));
     return MPRES_OK;
 }
 
@@ -594,11 +600,20 @@ int mpres_array_to_aos(mpres_ctx_t *c, void *dst, const mp_array_t *src, int cou
     return MPRES_OK;
 }
 
+// The variant of an element-wise call. Over 32 moduli a sum, which seldom rounds, keeps 8 lanes
+// a number where the built-in table gives one for the products (a sum of 10^6 in 0.135 ms with 8
+// lanes, 0.193 ms with one; a product of full operands in 4.6 and 0.66 ms).
+static const Ops *elem_ops(const mpres_ctx *c, int op, int count) {
+    const Ops *o = sized(c, OP_ELEM, count);
+    const bool sum = op == 0 || op == 1 || op == 4;
+    return c->host.n == 32 && sum && o->L == 1 && c->lt[OP_ELEM].builtin ? find_ops(32, 8) : o;
+}
+
 int mpres_elementwise(mpres_ctx_t *c, int op, int count, const void *x, const void *y, void *r, void *st) {
     if (!c || op < 0 || op > 4) return fail(MPRES_ERR_ARG, "invalid operation %d", op);
     if (count <= 0) return MPRES_OK;
     if (!x || !y || !r) return fail(MPRES_ERR_ARG, "null argument");
-    HIPCHK(sized(c, OP_ELEM, count)->elem(c->dev, op, count, (const char *)x, (const char *)y, (const double *)y,
+    HIPCHK(elem_ops(c, op, count)->elem(c->dev, op, count, (const char *)x, (const char *)y, (const double *)y,
                                           (char *)r, strm(st)));
     return MPRES_OK;
 }
@@ -1003,6 +1018,12 @@ size_t mpres_gemm_workspace(const mpres_ctx_t *c, int m, int n, int k) {
     return gemm_need(c, m, n, k) + (more ? more + 256 : 0);
 }
 
+// the variant of gemm's epilogue over mn entries: over 16 moduli its two products and a sum an
+// entry, which round when the operands are full, are element operations (sized(OP_ELEM))
+static const Ops *epilogue_ops(const mpres_ctx *c, const Ops *o, long long mn) {
+    return c->host.n == 16 ? sized(c, OP_ELEM, mn) : o;
+}
+
 int mpres_gemm(mpres_ctx_t *c, int ta, int tb, int m, int n, int k, const mp_array_t *alpha, const mp_array_t *A,
                int lda, const mp_array_t *B, int ldb, const mp_array_t *beta, mp_array_t *C, int ldc, void *ws,
                size_t wsb, void *st) {
@@ -1053,8 +1074,9 @@ int mpres_gemm(mpres_ctx_t *c, int ta, int tb, int m, int n, int k, const mp_arr
     }
     HIPCHK(fk.join());
     for (int pass = 2; pass < 5; pass++)
-        HIPCHK(o->gemm(c->dev, pass, c->bits, m, n, k, soa_of(alpha), soa_of(A), lda, soa_of(B), ldb, soa_of(beta),
-                       soa_of(C), ldc, w, ra, strm(st)));
+        HIPCHK((pass == 4 ? epilogue_ops(c, o, (long long)m * n) : o)
+                   ->gemm(c->dev, pass, c->bits, m, n, k, soa_of(alpha), soa_of(A), lda, soa_of(B), ldb, soa_of(beta),
+                          soa_of(C), ldc, w, ra, strm(st)));
     return MPRES_OK;
 }
 
@@ -1110,7 +1132,7 @@ int mpres_gemm_v2(mpres_ctx_t *c, int ta, int tb, int m, int n, int k, const voi
         if (pass == 3 && c->pos)
             HIPCHK(c->pos->gemm_v2(c->dev, tra, trb, m, n, k, (const char *)A, lda, (const char *)B, ldb, ra, rb, w,
                                    strm(st)));
-        HIPCHK(o->gemm_v2(c->dev, pass, c->bits, tra, trb, m, n, k, (const char *)alpha, (const char *)A,
+        HIPCHK((pass == 4 ? epilogue_ops(c, o, (long long)m * n) : o)->gemm_v2(c->dev, pass, c->bits, tra, trb, m, n, k, (const char *)alpha, (const char *)A,
                                         lda, (const char *)B, ldb, (const char *)beta, (char *)C, ldc, w, ra,
                                         pass == 0 ? fk.s1 : strm(st)));
     }
@@ -1362,7 +1384,7 @@ int mpres_batch_destroy(mpres_batch_t *b) {
 static int v1map(mpres_ctx_t *c, int op, int sf, int m, int n, const mp_array_t *S, int incs, const mp_array_t *X,
                  int ldx, int incx, const mp_array_t *Y, int ldy, int incy, mp_array_t *W, int ldw, int incw,
                  hipStream_t st) {
-    HIPCHK(c->ops[OP_ELEM]->v1map(c->dev, op, sf, m, n, S ? soa_of(S) : SoA{}, incs, soa_of(X), ldx, incx,
+    HIPCHK(sized(c, OP_ELEM, (long long)m * n)->v1map(c->dev, op, sf, m, n, S ? soa_of(S) : SoA{}, incs, soa_of(X), ldx, incx,
                                   Y ? soa_of(Y) : SoA{}, ldy, incy, soa_of(W), ldw, incw, st));
     return MPRES_OK;
 }
@@ -1675,7 +1697,7 @@ int mpres_set_lanes(mpres_ctx_t *c, int op, int lanes) {
     if (lanes == 0)
         install_builtin_lanes(c, op);
     else
-        c->lt[op].count = 0;
+        c->lt[op].count = 0, c->lt[op].builtin = false;
     return MPRES_OK;
 }
 
@@ -1697,6 +1719,7 @@ int mpres_set_lanes_table(mpres_ctx_t *c, int op, int count, const long long *bo
     }
     auto &t = c->lt[op];
     t.count = count;
+    t.builtin = false;
     for (int i = 0; i < count; i++) {
         t.bound[i] = bounds[i];
         t.ops[i] = ops[i];

@@ -230,49 +230,142 @@ MPH_HD void big_round(Big<W> &a, int &e, int p) {
     if (half && (sticky || (a.l[0] & 1u))) big_add_u32(a, 1u);
     e += sh;
 }
+// a top-aligned estimate: the leading 64 bits at and below limb W - 1 as a double
+template <int W>
+MPH_HD double big_top(const Big<W> &a) {
+    return fma((double)a.l[W - 1], 0x1p32, (double)a.l[W - 2]) + (double)a.l[W - 3] * 0x1p-32;
+}
+// r - d * b, 0 <= d < 2^26, in two's complement
+template <int W>
+MPH_HD void big_submul(Big<W> &r, const Big<W> &b, uint32_t d) {
+    uint64_t c = 0;
+    uint32_t borrow = 0;
+#pragma unroll
+    for (int i = 0; i < W; i++) {
+        c += (uint64_t)b.l[i] * d;
+        const uint64_t t = (uint64_t)r.l[i] - (uint32_t)c - borrow;
+        r.l[i] = (uint32_t)t;
+        borrow = (uint32_t)(t >> 63);
+        c >>= 32;
+    }
+}
+// a << S for a constant 0 < S < 32
+template <int S, int W>
+MPH_HD void big_shl_const(Big<W> &a) {
+#pragma unroll
+    for (int i = W - 1; i >= 0; i--) a.l[i] = (a.l[i] << S) | (i > 0 ? a.l[i - 1] >> (32 - S) : 0u);
+}
 // floor(a / b * 2^(q - 1)) for a, b of equal bit length L (so 1/2 < a/b < 2), with
-// W >= L + 2 bits: q restoring-division steps; returns the quotient and whether the
-// division left a remainder
+// W >= L + 2 bits, q <= 32 W; and whether the division left a remainder. Long division with
+// digits of BIG_DIGIT bits, each estimated in double from the leading bits (off by one at most) and corrected.
+constexpr int BIG_DIGIT = 24;
 template <int W>
 MPH_HD Big<W> big_div_bits(const Big<W> &a, const Big<W> &b, int q, bool &inexact) {
-    Big<W> r = a, quo;
+    // both operands at the top of limb W - 1, one limb of headroom
+    const int up = 32 * W - big_bitlen(b);
+    Big<W + 1> r = big_shl(big_widen<W + 1>(a), up), d = big_shl(big_widen<W + 1>(b), up);
+    const double inv = 1.0 / big_top(d);
+    Big<W> quo;
     big_zero(quo);
-    for (int i = 0; i < q; i++) {
-        quo = big_shl(quo, 1);
-        if (big_cmp(r, b) >= 0) {
-            big_sub(r, b);
-            quo.l[0] |= 1u;
-        }
-        r = big_shl(r, 1);
+    if (big_cmp(r, d) >= 0) {
+        big_sub(r, d);
+        quo.l[0] = 1u;
     }
-    inexact = !big_is_zero(r);
+    const int digits = (q - 1 + BIG_DIGIT - 1) / BIG_DIGIT, extra = digits * BIG_DIGIT - (q - 1);
+    bool lost = false;
+#pragma nounroll
+    for (int i = 0; i < digits; i++) {
+        big_shl_const<BIG_DIGIT>(r);
+        int t = (int)(big_top(r) * inv);
+        big_submul(r, d, (uint32_t)t);
+        if ((int)r.l[W] < 0) {  // one too many
+            big_add(r, d);
+            t--;
+        } else if (big_cmp(r, d) >= 0) {
+            big_sub(r, d);
+            t++;
+        }
+        if (i + 1 < digits) {
+            big_shl_const<BIG_DIGIT>(quo);
+            quo.l[0] |= (uint32_t)t;
+        } else {  // the last digit's bits below 2^-(q - 1) only tell whether there is a remainder
+            quo = big_shl(quo, BIG_DIGIT - extra);
+            quo.l[0] |= (uint32_t)t >> extra;
+            lost = ((uint32_t)t & ((1u << extra) - 1u)) != 0;
+        }
+    }
+    inexact = lost || !big_is_zero(r);
     return quo;
 }
-// s = floor(sqrt(a)) by the digit-by-digit method; inexact when s^2 != a
+// s = floor(sqrt(a)), a below 2^(32 W - 48); inexact when s^2 != a. The root's digits of 24 bits: the
+// first from a's leading 47 or 48 bits in double, each further one d from the remainder r
+// (next two digits of a appended): the largest with d (2 s + d) <= r, estimated as r / (2 s) and
+// corrected.
 template <int W>
 MPH_HD Big<W> big_isqrt(const Big<W> &a, bool &inexact) {
-    Big<W> num = a, res, bit, t;
-    big_zero(res);
-    big_zero(bit);
-    const int b = big_bitlen(a);
-    if (b == 0) {
+    Big<W> s;
+    big_zero(s);
+    const int len = big_bitlen(a);
+    if (len == 0) {
         inexact = false;
-        return res;
+        return s;
     }
-    const int top = (b - 1) & ~1;  // highest even bit position not above a's leading bit
-    bit.l[top >> 5] = 1u << (top & 31);
-    for (int i = top; i >= 0; i -= 2) {
-        t = res;
-        big_add(t, bit);
-        res = big_shr(res, 1);
-        if (big_cmp(num, t) >= 0) {
-            big_sub(num, t);
-            big_add(res, bit);
+    // a 4^z, of 48 digits - 1 or 48 digits bits, at the top of x: its 48-bit digits are taken from
+    // there in turn, and the root comes out times 2^z
+    const int digits = (len + 47) / 48, z = (48 * digits - len) / 2;
+    Big<W> x = big_shl(a, 32 * W - 48 * digits + 2 * z);
+    auto next = [&]() -> uint64_t {
+        const uint64_t v = ((uint64_t)x.l[W - 1] << 16) | (x.l[W - 2] >> 16);
+        big_shl_const<24>(x);
+        big_shl_const<24>(x);
+        return v;
+    };
+    uint64_t c = next();
+    uint64_t s0 = (uint64_t)sqrt((double)c);
+    Big<W> r;  // remainder, at most 2 s
+    big_zero(r);
+    r.l[0] = (uint32_t)(c - s0 * s0);
+    r.l[1] = (uint32_t)((c - s0 * s0) >> 32);
+    s.l[0] = (uint32_t)s0;
+#pragma nounroll
+    for (int i = 1; i < digits; i++) {
+        c = next();
+        big_shl_const<24>(r);
+        big_shl_const<24>(r);
+        r.l[0] |= (uint32_t)c;
+        r.l[1] |= (uint32_t)(c >> 32);
+        big_shl_const<24>(s);
+        const Big<W> s2 = big_shl(s, 1);
+        // estimate from the leading bits of 2 s
+        const int k = big_bitlen(s2) > 64 ? big_bitlen(s2) - 64 : 0;
+        const Big<W> st = big_shr(s2, k), rt = big_shr(r, k);
+        const double sd = fma((double)st.l[1], 0x1p32, (double)st.l[0]);
+        const double rd = fma(fma((double)rt.l[2], 0x1p32, (double)rt.l[1]), 0x1p32, (double)rt.l[0]);
+        double e = rd / sd;
+        e = e > 16777215.0 ? 16777215.0 : e;
+        uint32_t d = (uint32_t)e;
+        // r - d (2 s + d)
+        Big<W> t = s2;
+        t.l[0] |= d;  // 2 s is a multiple of 2^25
+        big_submul(r, t, d);
+        for (int j = 0; j < 2 && (int)r.l[W - 1] < 0; j++) {  // too many: add back (2 s + 2 d - 1)
+            d--;
+            Big<W> u = s2;
+            big_add_u32(u, 2 * d + 1);
+            big_add(r, u);
         }
-        bit = big_shr(bit, 2);
+        {  // one too few: r >= 2 s + 2 d + 1
+            Big<W> u = s2;
+            big_add_u32(u, 2 * d + 1);
+            if (d < 16777215u && big_cmp(r, u) >= 0) {
+                big_sub(r, u);
+                d++;
+            }
+        }
+        s.l[0] |= d;
     }
-    inexact = !big_is_zero(num);
-    return res;
+    inexact = !big_is_zero(r) || big_any_below(s, z);
+    return big_shr(s, z);
 }
 
 }  // namespace mph

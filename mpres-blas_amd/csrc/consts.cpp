@@ -82,6 +82,11 @@ bool compute_consts(const ModuliSet &s, DevConsts &c, std::vector<int> &pow2) {
         c.md[i] = (double)s.m[i];
         c.minv[i] = 1.0 / (double)s.m[i];
     }
+    c.mus = 31 - __builtin_clz((unsigned)s.m[0]);
+    for (int i = 0; i < n; i++) {
+        if (31 - __builtin_clz((unsigned)s.m[i]) != c.mus) return false;  // moduli of one set have one bit length
+        c.mu[i] = (uint32_t)(((uint64_t)1 << (c.mus + 32)) / (uint32_t)s.m[i]);
+    }
     // M in 32-bit limbs
     std::vector<uint32_t> M(1, 1u);
     for (int i = 0; i < n; i++) {
@@ -107,11 +112,15 @@ bool compute_consts(const ModuliSet &s, DevConsts &c, std::vector<int> &pow2) {
             if (j != i) p = (p * (s.m[j] % s.m[i])) % s.m[i];
         c.w[i] = (int)inverse_mod(p, s.m[i]);
     }
-    pow2.assign((size_t)(s.log2m + 1) * n, 0);
+    const size_t rows = (size_t)s.log2m + 1;
+    const auto quot = [&](int v, int i) { return (uint32_t)(((uint64_t)(uint32_t)v << 32) / (uint32_t)s.m[i]); };
+    for (int i = 0; i < n; i++) c.wq[i] = quot(c.w[i], i);
+    pow2.assign(2 * rows * n, 0);
     for (int j = 0; j < n; j++) {
         int64_t v = 1;
         for (int i = 0; i <= s.log2m; i++) {
             pow2[(size_t)i * n + j] = (int)v;
+            pow2[(rows + i) * n + j] = (int)quot((int)v, j);
             v = (v * 2) % s.m[j];
         }
     }
@@ -128,6 +137,7 @@ bool compute_consts(const ModuliSet &s, DevConsts &c, std::vector<int> &pow2) {
             int64_t q = 1;
             for (int k = 0; k <= i; k++) q = (q * 2) % s.m[j];
             c.pow2inv[i][j] = (int)inverse_mod(q, s.m[j]);
+            c.pow2invq[i][j] = quot(c.pow2inv[i][j], j);
         }
     }
     for (int i = 0; i < n; i++)
@@ -168,16 +178,29 @@ bool compute_consts(const ModuliSet &s, DevConsts &c, std::vector<int> &pow2) {
         c.rrd[i] = emu_div_rd(1.0, (double)s.m[i]);
         c.rru[i] = emu_div_ru(1.0, (double)s.m[i]);
     }
-    // limbs of M and of M / m_i, powers of 2^16 modulo m_i
+    // limbs of M, -M and M / m_i, powers of 2^16 modulo m_i
     {
-        const auto limb16 = [](const std::vector<uint32_t> &v, int l) {
-            return l / 2 < (int)v.size() ? (double)((v[l / 2] >> (16 * (l & 1))) & 0xffffu) : 0.0;
+        const auto limb28 = [](const std::vector<uint32_t> &v, int l) {
+            uint32_t r = 0;
+            for (int b = 0; b < 28; b++) {
+                const size_t p = 28 * (size_t)l + b;
+                if (p / 32 < v.size()) r |= ((v[p / 32] >> (p % 32)) & 1u) << b;
+            }
+            return r;
         };
         double pm = 0;
         for (size_t i = M.size(); i-- > 0;) pm = pm * 4294967296.0 + (double)M[i];
         c.pmod = pm;
         c.pinv = 1.0 / pm;
-        for (int l = 0; l < 2 * n; l++) c.m16[l] = limb16(M, l);
+        std::vector<uint32_t> neg(2 * MAXN, 0u);
+        uint64_t carry = 1;
+        for (size_t i = 0; i < neg.size(); i++) {
+            const uint64_t t = (uint64_t)(uint32_t)~(i < M.size() ? M[i] : 0u) + carry;
+            neg[i] = (uint32_t)t;
+            carry = t >> 32;
+        }
+        for (int l = 0; l < MAXN; l++) c.m32[l] = l < (int)M.size() ? M[l] : 0u;
+        for (int l = 0; l < P28; l++) c.mn28[l] = limb28(neg, l);
         for (int j = 0; j < n; j++) {
             std::vector<uint32_t> Q(M);
             uint64_t rem = 0;
@@ -186,10 +209,10 @@ bool compute_consts(const ModuliSet &s, DevConsts &c, std::vector<int> &pow2) {
                 Q[i] = (uint32_t)(t / (uint32_t)s.m[j]);
                 rem = t % (uint32_t)s.m[j];
             }
+            for (int l = 0; l < P28; l++) c.mi28[l][j] = limb28(Q, l);
             int64_t q = 1;
-            for (int l = 0; l < 2 * n; l++) {
-                c.mi16[l][j] = limb16(Q, l);
-                c.q16[l][j] = (double)q;
+            for (int l = 0; l < MAXN; l++) {
+                c.q16[j][l] = (double)q;
                 q = (q << 16) % s.m[j];
             }
         }

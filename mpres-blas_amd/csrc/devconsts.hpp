@@ -11,6 +11,7 @@
 namespace mph {
 
 constexpr int MAXN = 32;
+constexpr int P28 = (32 * MAXN + 27) / 28;  // 28-bit limbs of a number below M
 constexpr int P2T = 30;  // RNS_P2_SCALING_THRESHOLD (src/params.h)
 
 struct ErC {
@@ -39,12 +40,18 @@ struct DevConsts {
     int h[P2T][MAXN];      // M_i mod 2^(j+1)
     int pow2inv[P2T][MAXN];// 2^-(j+1) mod m_i
     int mrcinv[MAXN][MAXN];// m_i^-1 mod m_j (j > i)
-    // positional form (pos.hpp), 16-bit limbs as doubles, least significant first
+    // positional integers (posint.hpp), least significant limb first
     double pinv, pmod;               // 1 / M and M, rounded
-    double mi16[2 * MAXN][MAXN];     // limb l of M / m_i
-    double m16[2 * MAXN];            // limb l of M
-    double q16[2 * MAXN][MAXN];      // 2^(16 l) mod m_i
-    const int *pow2;       // device pointer: RNS_POW2, (log2m + 1) x n, row-major
+    uint32_t mi28[P28][MAXN];        // 28-bit limb l of M / m_i
+    uint32_t mn28[P28];              // 28-bit limb l of -M (two's complement)
+    uint32_t m32[MAXN];              // word l of M
+    double q16[MAXN][MAXN];          // [i][l]: 2^(16 l) mod m_i
+    uint32_t mu[MAXN];     // floor(2^(mus + 32) / m_i) (mulmod_i)
+    int mus;               // bit length of the moduli, less one
+    // floor(v 2^32 / m_i) for the fixed factors v above (mulmod_c)
+    uint32_t wq[MAXN], pow2invq[P2T][MAXN];
+    // device pointer: RNS_POW2, (log2m + 1) x n, row-major, then the same shape of floor(v 2^32 / m_i)
+    const int *pow2;
 };
 
 }  // namespace mph

@@ -29,6 +29,7 @@
 #include "devconsts.hpp"
 #include "numerics.hpp"
 #include "ops.hpp"
+#include "posint.hpp"
 #include "rare.hpp"
 
 namespace mph {
@@ -190,21 +191,48 @@ __device__ __forceinline__ bool sc_fma_step(const ScC &C, Sc &acc, int xs, int x
     return sc_add_step(C, acc, p);
 }
 
+// the rounding of a number held by one lane, out of line (rare at 16 and 32 moduli)
+template <int N>
+__device__ __noinline__ void ool_pos_round(const DevConsts *C, int *d, int *exp, Er *ev0, Er *ev1) {
+    int e = *exp, t[N];
+    Er a = *ev0, b = *ev1;
+#pragma unroll
+    for (int i = 0; i < N; i++) t[i] = d[i];
+    if (!pos_round<N>(C, t, e, a, b)) {
+        Core<N, 1> k{C, C->pow2, 0};
+        k.load();
+        ool_round<N, 1>(k, d, exp, ev0, ev1);
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < N; i++) d[i] = t[i];
+    *exp = e;
+    *ev0 = a;
+    *ev1 = b;
+}
+
+// element kernels that round in a function of their own (Grp::round_fails). With more lanes a
+// number that function, run by one lane of the group, leaves the others idle: over 32 moduli and
+// 10^6 full products 8 lanes took 3.5 ms with it, one lane 0.66
+constexpr bool cold_round(int N, int L) { return (N == 16 && L <= 2) || (N > 16 && L == 1); }
+
 template <int N, int L>
 struct Grp {
     static_assert(N % L == 0, "L must divide N");
     static_assert((L & (L - 1)) == 0 && L <= 32, "L must be a power of two <= 32");
     static constexpr int R = N / L;
-    static constexpr bool INL = (N <= 8);               // rare paths inlined and unrolled
+    static constexpr bool INL = (N <= 8 || R == 1);     // rare paths inlined and unrolled
     static constexpr bool CACHE = (L > 1 && R <= 8);    // per-lane moduli kept in registers
     static constexpr int CR = CACHE ? R : 1;
 
     Core<N, L> k;
     double cmd[CR], cmv[CR];
     int cmi[CR];
+    uint32_t cmu[CR];
+    int mus;
     ScC K;  // constants of the scalar steps, read once
 
-    __device__ __forceinline__ explicit Grp(const DevConsts *c) : K(sc_consts(c)) {
+    __device__ __forceinline__ explicit Grp(const DevConsts *c) : mus(c->mus), K(sc_consts(c)) {
         k.C = c;
         k.P2 = c->pow2;
         k.lane = (int)(__lane_id() & (L - 1));
@@ -215,6 +243,7 @@ struct Grp {
                 cmd[r] = c->md[ix(r)];
                 cmv[r] = c->minv[ix(r)];
                 cmi[r] = c->m[ix(r)];
+                cmu[r] = c->mu[ix(r)];
             }
         }
     }
@@ -232,7 +261,11 @@ struct Grp {
         if constexpr (CACHE) return cmi[r];
         else return k.C->m[ix(r)];
     }
-    __device__ __forceinline__ int mmul(int a, int b, int r) const { return mulmod(a, b, md(r), mv(r)); }
+    __device__ __forceinline__ uint32_t mu(int r, const DevConsts *c) const {
+        if constexpr (CACHE) return cmu[r];
+        else return c->mu[ix(r)];
+    }
+    __device__ __forceinline__ int mmul(int a, int b, int r) const { return mmul(a, b, r, k.C); }
     // Moduli read through a pointer the compiler must treat as new on every call
     // (HINT): keeps the fast kernels' multiply-accumulate loops from hoisting N
     // moduli and reciprocals into registers (they are re-read from the scalar
@@ -258,7 +291,7 @@ struct Grp {
         else return c->m[ix(r)];
     }
     __device__ __forceinline__ int mmul(int a, int b, int r, const DevConsts *c) const {
-        return mulmod(a, b, md(r, c), mv(r, c));
+        return mulmod_i((uint32_t)a, (uint32_t)b, (uint32_t)mi(r, c), mu(r, c), mus);
     }
     __device__ __forceinline__ int prow(int g) const { return g > k.C->log2m ? k.C->log2m : g; }
     __device__ __forceinline__ Er unit_low() const { return Er{k.C->unit_low.frac, k.C->unit_low.exp}; }
@@ -279,7 +312,10 @@ struct Grp {
                 Er e0 = a.ev0, e1 = a.ev1;
 #pragma unroll
                 for (int r = 0; r < R; r++) t[r] = a.d[r];
-                ool_round<N, L>(k, t, &e, &e0, &e1);
+                if constexpr (L == 1)
+                    ool_pos_round<N>(k.C, t, &e, &e0, &e1);
+                else
+                    ool_round<N, L>(k, t, &e, &e0, &e1);
 #pragma unroll
                 for (int r = 0; r < R; r++) a.d[r] = t[r];
                 a.exp = e;
@@ -287,6 +323,38 @@ struct Grp {
                 a.ev1 = e1;
             }
         }
+    }
+    // round_if_needed for the element kernels, whose operations leave it out (RND = false): with
+    // one lane per number over 16 and 32 moduli it is inlined, under the kernel's own register
+    // budget (ELEM_WAVES)
+    __device__ __forceinline__ void round_here(MP<R> &a) const {
+        if constexpr (!INL && L == 1) {
+            if (needs_round(a) && !pos_round<N>(k.C, a.d, a.exp, a.ev0, a.ev1)) {
+                int t[R], e = a.exp;  // memory of their own: the number stays in registers
+                Er e0 = a.ev0, e1 = a.ev1;
+#pragma unroll
+                for (int r = 0; r < R; r++) t[r] = a.d[r];
+                ool_round<N, 1, true>(k, t, &e, &e0, &e1);
+#pragma unroll
+                for (int r = 0; r < R; r++) a.d[r] = t[r];
+                a.exp = e;
+                a.ev0 = e0;
+                a.ev1 = e1;
+            }
+        } else {
+            round_if_needed(a);
+        }
+    }
+    // Element kernels that cold_round names compute without rounding first (COLD = false: true if
+    // the number needs it) and do a number whose results need it again, from its operands, in a
+    // function of its own (COLD = true); elsewhere the number is rounded in place. Inlined, the
+    // rounding's registers slowed the numbers that need none (axpy of 10^6 numbers of 212 bits
+    // 0.066 ms, now 0.063); the second pass over the operands costs the full ones (0.23 ms, now 0.26).
+    template <bool COLD>
+    __device__ __forceinline__ bool round_fails(MP<R> &a) const {
+        if constexpr (cold_round(N, L) && !COLD) return needs_round(a);
+        round_here(a);
+        return false;
     }
     // full interval evaluation of a number's residues (rns_eval_compute, CUDA)
     __device__ __forceinline__ void eval_full(const int *d, Er &lo, Er &up) const {
@@ -389,18 +457,28 @@ struct Grp {
         return align(x.sign, x.exp, x.ev0, x.ev1, y.sign, y.exp, y.ev0, y.ev1);
     }
 
-    // residue of (2^gamma x fx + 2^theta y fy) mod m for one residue (at most one shift is nonzero)
-    __device__ __forceinline__ int combine(int xd, int yd, const int *row, bool shx, bool sh, int fs, int fo,
-                                          int sign, int r, const DevConsts *c) const {
+    // -t mod m for 0 <= t < m
+    __device__ __forceinline__ static uint32_t negmod(uint32_t t, uint32_t m) {
+        const uint32_t a = m - t, z = 0u - t;  // t = 0: z
+        return a < z ? a : z;
+    }
+    // residue of (2^gamma x fx + 2^theta y fy) mod m for one residue (at most one shift, sh, is
+    // nonzero; row: its row of RNS_POW2); the residue of the magnitude when sign is set
+    __device__ __forceinline__ int combine(int xd, int yd, int row, bool shx, bool sh, int fs, int fo, int sign, int r,
+                                          const DevConsts *c) const {
+        const uint32_t m = (uint32_t)mi(r, c);
         const int sv = shx ? xd : yd;
-        const int ov = shx ? yd : xd;
-        const int t = sh ? mmul(sv, row[ix(r)], r, c) : sv;
-        const double v = mod_fix((double)fs * (double)t + (double)fo * (double)ov, md(r, c));
-        const int vi = (int)v;
-        return sign ? (vi != 0 ? mi(r, c) - vi : 0) : vi;
+        const uint32_t ov = (uint32_t)(shx ? yd : xd);
+        // one table entry a residue where a lane holds several: its reads of a row that no other
+        // lane reads cost more than the three instructions that the quotient table saves
+        const uint32_t t = (uint32_t)(!sh ? sv : R > 1 ? mmul(sv, k.P2[(size_t)row * N + ix(r)], r, c) : k.xpow2(sv, row, r, m));
+        const uint32_t u = fs > 0 ? t : fs < 0 ? negmod(t, m) : 0u, w = fo > 0 ? ov : fo < 0 ? negmod(ov, m) : 0u;
+        const uint32_t v = u + w, q = v - m, z = v < q ? v : q;
+        return (int)(sign ? negmod(z, m) : z);
     }
 
     // cuda::mp_add (mp_add_common + rounding), src/arith/add.cuh:126-200
+    template <bool RND = true>
     __device__ __forceinline__ void add(MP<R> &res, const MP<R> &x, const MP<R> &y) const {
         const Align a = align(x, y);
         Er e0, e1;
@@ -416,12 +494,13 @@ struct Grp {
         }
         const bool shx = a.gamma > 0;
         const int sh = a.gamma + a.theta;
-        const int *row = k.P2 + (size_t)prow(sh) * N;
+        const int row = prow(sh);
         const int fs = shx ? a.fx : a.fy, fo = shx ? a.fy : a.fx;
 #pragma unroll
         for (int r = 0; r < R; r++) res.d[r] = combine(x.d[r], y.d[r], row, shx, sh != 0, fs, fo, sign, r, k.C);
-        finish_add(res, a, e0, e1, sign);
+        finish_add<RND>(res, a, e0, e1, sign);
     }
+    template <bool RND>
     __device__ __forceinline__ void finish_add(MP<R> &res, const Align &a, Er e0, Er e1, int sign) const {
         res.sign = sign;
         res.exp = (a.ex == 0) ? a.ey : a.ex;
@@ -432,7 +511,7 @@ struct Grp {
             res.ev0 = e0;
             res.ev1 = e1;
         }
-        round_if_needed(res);
+        if constexpr (RND) round_if_needed(res);
     }
 
     // scalar part of cuda::mp_mul (mp_mul_common, src/arith/mul.cuh:35-42)
@@ -446,11 +525,12 @@ struct Grp {
         res.ev1 = p.ev1;
     }
     // cuda::mp_mul, src/arith/mul.cuh:53-74
+    template <bool RND = true>
     __device__ __forceinline__ void mul(MP<R> &res, const MP<R> &x, const MP<R> &y) const {
         mul_scalars(res, x.sign, x.exp, x.ev0, x.ev1, y.sign, y.exp, y.ev0, y.ev1);
 #pragma unroll
         for (int r = 0; r < R; r++) res.d[r] = mmul(x.d[r], y.d[r], r);
-        round_if_needed(res);
+        if constexpr (RND) round_if_needed(res);
     }
 
     // scalar part of cuda::mp_mul_d (src/arith/muld.cuh:59-67); returns the significand of y
@@ -465,11 +545,12 @@ struct Grp {
         return sig;
     }
     // cuda::mp_mul_d, src/arith/muld.cuh:59-73
+    template <bool RND = true>
     __device__ __forceinline__ void mul_d(MP<R> &res, const MP<R> &x, double y) const {
         const double sig = muld_scalars(res, x.sign, x.exp, x.ev0, x.ev1, y);
 #pragma unroll
         for (int r = 0; r < R; r++) res.d[r] = mmul(x.d[r], modd(sig, md(r), mv(r)), r);
-        round_if_needed(res);
+        if constexpr (RND) round_if_needed(res);
     }
 
     // acc = acc + x[ix] * y[iy] (mp_mul then mp_add with the reference's rounding),
@@ -542,7 +623,7 @@ struct Grp {
         }
         const bool shx = a.gamma > 0;
         const int sh = a.gamma + a.theta;
-        const int *row = k.P2 + (size_t)prow(sh) * N;
+        const int row = prow(sh);
         const int fs = shx ? a.fx : a.fy, fo = shx ? a.fy : a.fx;
         const DevConsts *c = fresh<!FULL>();
 #pragma unroll
@@ -577,7 +658,7 @@ struct Grp {
             if (sign != (e1.frac < 0)) return false;
             const bool shx = a.gamma > 0;
             const int sh = a.gamma + a.theta;
-            const int *row = k.P2 + (size_t)prow(sh) * N;
+            const int row = prow(sh);
             const int fs = shx ? a.fx : a.fy, fo = shx ? a.fy : a.fx;
             const DevConsts *c = fresh<!FULL>();
 #pragma unroll
@@ -597,6 +678,7 @@ struct Grp {
 
     // v1 element-wise addition: esi + digits + round kernels, src/mpvector.cuh:234-472, 669-714
     // (no MRC on a straddling interval; residues via a double-reciprocal quotient)
+    template <bool RND = true>
     __device__ __forceinline__ void vadd(MP<R> &res, const MP<R> &x, const MP<R> &y) const {
         const Align a = align(x, y);
         Er e0, e1;
@@ -637,7 +719,7 @@ struct Grp {
             }
             res.d[r] = v < 0 ? v + mi(r) : v;
         }
-        if ((res.ev1.exp - k.C->mp_h + 1) * (res.ev1.frac != 0) > 0) round_if_needed(res);
+        if constexpr (RND) round_if_needed(res);
     }
 
     // mp_set_d, src/arith/assign.cuh:54-81, with the CUDA interval evaluation
@@ -661,6 +743,10 @@ struct Grp {
         // X < 2^53 <= m_0 ... m_{N-2} for every supported set, so mrd(X) = 0
         if constexpr (INL) {
             rns_eval<N, L, true, true>(k, res.d, res.ev0, res.ev1, true);
+        } else if constexpr (L == 1) {
+            // (the full evaluation differs from it only where sumu >= acc, for X above M / 2^23)
+            uint32_t t[Pos<N>::W] = {(uint32_t)sig, (uint32_t)(sig >> 32)};
+            pos_eval_fast<N>(k.C, t, res.ev0, res.ev1);
         } else {
             int t[R];
             Er a, b;
@@ -670,7 +756,7 @@ struct Grp {
             res.ev0 = a;
             res.ev1 = b;
         }
-        round_if_needed(res);
+        round_here(res);
     }
 };
 

@@ -18,6 +18,7 @@
 #include "bigint.hpp"
 #include "devconsts.hpp"
 #include "numerics.hpp"
+#include "posint.hpp"
 
 namespace mph {
 
@@ -46,6 +47,12 @@ __device__ __forceinline__ int e_mod_mul(int x, int y, int m, double d) {
     const long long r = (long long)x * (long long)y;
     const int q = (int)((double)r * d);
     return (int)(r - (long long)q * (long long)m);
+}
+// a / m rounded to nearest from minv = RN(1 / m): Markstein's correction of RN(a minv) by the
+// exact remainder
+__device__ __forceinline__ double e_quot(double a, double m, double minv) {
+    const double q = a * minv;
+    return fma(fma(-q, m, a), minv, q);
 }
 // last mixed-radix digit, src/rns.cuh:495-520 (exact)
 template <int N>
@@ -103,14 +110,14 @@ __device__ void cpu_eval(const DevConsts *__restrict__ C, const int *x, Er &low,
 #pragma unroll
         for (int i = 0; i < N; i++) {
             s[i] = e_mod_mul(s[i], C->pow2[(size_t)k * N + i], C->m[i], C->minv[i]);
-            fu[i] = e_widen((double)s[i] / C->md[i], true);
+            fu[i] = e_widen(e_quot((double)s[i], C->md[i], C->minv[i]), true);
         }
         sumu = e_psum<N>(fu, true);
         sumu -= (unsigned)sumu;
         K += k;
     }
 #pragma unroll
-    for (int i = 0; i < N; i++) fl[i] = e_widen((double)s[i] / C->md[i], false);
+    for (int i = 0; i < N; i++) fl[i] = e_widen(e_quot((double)s[i], C->md[i], C->minv[i]), false);
     suml = e_psum<N>(fl, false);
     suml -= (unsigned)suml;
     low = er_set_d(suml);
@@ -129,28 +136,15 @@ constexpr int big_limbs() {
 template <int N>
 using BigN = Big<big_limbs<N>()>;
 
-// X of a number's residues (0 <= X < M), mixed-radix conversion then Horner's rule
+// X of a number's residues (0 <= X < M; residues outside [0, m_i) are reduced first)
 template <int N>
 __device__ BigN<N> residues_to_big(const DevConsts *__restrict__ C, const int *d) {
     int a[N];
 #pragma unroll
-    for (int i = 0; i < N; i++) {
-        const int m = C->m[i];
-        const int v = d[i] % m;
-        a[i] = v < 0 ? v + m : v;
-    }
-#pragma unroll
-    for (int j = 0; j < N - 1; j++)
-#pragma unroll
-        for (int i = j + 1; i < N; i++) {
-            int t = a[i] - a[j];
-            t = t < 0 ? t + C->m[i] : t;
-            a[i] = mulmod(t, C->mrcinv[j][i], C->md[i], C->minv[i]);
-        }
+    for (int i = 0; i < N; i++) a[i] = pos_reduce(d[i], C->m[i]);
     BigN<N> X;
     big_zero(X);
-    X.l[0] = (uint32_t)a[N - 1];
-    for (int i = N - 2; i >= 0; i--) big_mul_add_u32(X, (uint32_t)C->m[i], (uint32_t)a[i]);
+    pos_from_digits<N, N, false>(C, a, X.l);
     return X;
 }
 
@@ -173,7 +167,10 @@ __device__ void big_to_mp(const DevConsts *__restrict__ C, BigN<N> Q, int e, int
     Q = big_shr(Q, tz);
     oexp = e + tz;
 #pragma unroll
-    for (int i = 0; i < N; i++) digits[i] = (int)big_mod_u32(Q, (uint32_t)C->m[i]);
+    for (int i = 0; i < N; i++) {
+        digits[i] = pos_residue<N, Pos<N>::W>(C, Q.l, i);  // at most MP_PRECISION + 1 bits
+        if (i % 2 == 1) pos_fence();
+    }
     cpu_eval<N>(C, digits, lo, up);
 }
 

@@ -33,6 +33,17 @@
 namespace mph {
 
 constexpr int BLK = 256;
+// Element kernels with one lane per number over 16 and 32 moduli are held to three (two) waves
+// per SIMD, which is what the positional rounding needs to keep its integers in registers: inlined
+// in the kernel (ELEM_WAVES), or in the function that does a number again (COLD_WAVES,
+// Grp::round_fails).
+#if defined(__HIPCC__)
+#define ELEM_WAVES(N, L) __attribute__((amdgpu_waves_per_eu(((N) > 8 && (L) == 1) ? ((N) == 16 ? 3 : 2) : 1)))
+#define COLD_WAVES(N, L) __attribute__((amdgpu_waves_per_eu(cold_round(N, L) ? ((N) == 16 ? 3 : 2) : 1)))
+#else
+#define ELEM_WAVES(N, L)
+#define COLD_WAVES(N, L)
+#endif
 constexpr int REDO = 2;  // sign of a workspace result whose chain the fixup kernel recomputes
 
 
@@ -108,7 +119,7 @@ __device__ __forceinline__ long long group_id() {
 // ---------------------------------------------------------------- conversion
 // mp_set_d for count doubles; out either SoA (soa_out) or AoS
 template <int N, int L, bool SOA_OUT>
-__global__ __launch_bounds__(BLK) void k_set_d(const DevConsts *__restrict__ C, const double *__restrict__ x, int count,
+__global__ __launch_bounds__(BLK) ELEM_WAVES(N, L) void k_set_d(const DevConsts *__restrict__ C, const double *__restrict__ x, int count,
                                                SoA so, AoSRef<N> ao) {
     so = rd(so);
     const long long i = group_id<L>();
@@ -135,8 +146,7 @@ __device__ __forceinline__ int exp_of(const AoSRef<N> &v, long long i) { return 
 // ---------------------------------------------------------------- export
 // The integer X (0 <= X < M) that a number's residues stand for, as the reference's
 // mp_get_d / mp_get_mpfr form it (src/arith/assign.cuh:154-211, CRT with the orthogonal
-// base, mod M): here by mixed-radix conversion, X = a_0 + a_1 m_0 + a_2 m_0 m_1 + ...,
-// then Horner's rule over 32-bit limbs, least significant first. Residues outside
+// base, mod M; pos_from_digits): 32-bit limbs, least significant first. Residues outside
 // [0, m_i) are reduced first. One thread per number, loops unrolled (arrays in registers).
 template <int N>
 constexpr int export_limbs() {
@@ -144,36 +154,12 @@ constexpr int export_limbs() {
 }
 template <int N>
 __device__ __forceinline__ void mp_integer(const DevConsts *__restrict__ C, const int *d, uint32_t *X) {
-    constexpr int LW = export_limbs<N>();
     int a[N];
 #pragma unroll
-    for (int i = 0; i < N; i++) {
-        const int m = C->m[i];
-        int v = d[i] % m;
-        a[i] = v < 0 ? v + m : v;
-    }
+    for (int i = 0; i < N; i++) a[i] = pos_reduce(d[i], pos_const(C->m[i]));
+    pos_from_digits<N, N, false>(C, a, X);
 #pragma unroll
-    for (int j = 0; j < N - 1; j++)
-#pragma unroll
-        for (int i = j + 1; i < N; i++) {
-            int t = a[i] - a[j];
-            t = t < 0 ? t + C->m[i] : t;
-            a[i] = mulmod(t, C->mrcinv[j][i], C->md[i], C->minv[i]);
-        }
-#pragma unroll
-    for (int l = 0; l < LW; l++) X[l] = 0;
-    X[0] = (uint32_t)a[N - 1];
-#pragma unroll
-    for (int i = N - 2; i >= 0; i--) {
-        uint64_t carry = (uint64_t)a[i];
-        const uint64_t m = (uint64_t)C->m[i];
-#pragma unroll
-        for (int l = 0; l < LW; l++) {
-            const uint64_t t = (uint64_t)X[l] * m + carry;
-            X[l] = (uint32_t)t;
-            carry = t >> 32;
-        }
-    }
+    for (int l = N; l < export_limbs<N>(); l++) X[l] = 0;
 }
 // (-1)^sign X 2^exp as a double: X rounded to 53 significant bits to nearest (ties to
 // even), then scaled by a power of two with one more rounding to nearest when the result
@@ -310,27 +296,37 @@ __global__ __launch_bounds__(BLK) void k_sqrt(const DevConsts *__restrict__ C, i
 }
 
 // ---------------------------------------------------------------- element-wise
-template <int N, int L, int OP>
-__global__ __launch_bounds__(BLK) void k_elem(const DevConsts *__restrict__ C, int count, AoSRef<N> x, AoSRef<N> y,
-                                              const double *__restrict__ yd, AoSRef<N> r) {
-    const long long i = group_id<L>();
-    if (i >= count) return;
+template <int N, int L, int OP, bool COLD>
+__device__ __forceinline__ bool elem_one(const DevConsts *__restrict__ C, AoSRef<N> x, AoSRef<N> y,
+                                         const double *__restrict__ yd, AoSRef<N> r, long long i) {
     Grp<N, L> g(C);
     MP<N / L> a, b, c;
     load_aos(g, a, x, i);
     if (OP == 3) {
-        g.mul_d(c, a, yd[i]);
+        g.template mul_d<false>(c, a, yd[i]);
     } else {
         load_aos(g, b, y, i);
-        if (OP == 0) g.add(c, a, b);
-        if (OP == 1) {
-            b.sign ^= 1;  // mp_sub, src/arith/sub.cuh:41-53
-            g.add(c, a, b);
-        }
-        if (OP == 2) g.mul(c, a, b);
-        if (OP == 4) g.vadd(c, a, b);
+        if (OP == 1) b.sign ^= 1;  // mp_sub, src/arith/sub.cuh:41-53
+        if (OP < 2) g.template add<false>(c, a, b);
+        if (OP == 2) g.template mul<false>(c, a, b);
+        if (OP == 4) g.template vadd<false>(c, a, b);
     }
+    if (g.template round_fails<COLD>(c)) return g.lane() == 0;
     store_aos(g, c, r, i);
+    return false;
+}
+template <int N, int OP>
+__device__ __noinline__ void elem_rounded(const DevConsts *C, AoSRef<N> x, AoSRef<N> y, const double *yd, AoSRef<N> r,
+                                          long long i) {
+    elem_one<N, 1, OP, true>(uniform_ptr(C), x, y, yd, r, i);
+}
+template <int N, int L, int OP>
+__global__ __launch_bounds__(BLK) COLD_WAVES(N, L) void k_elem(const DevConsts *__restrict__ C, int count, AoSRef<N> x, AoSRef<N> y,
+                                              const double *__restrict__ yd, AoSRef<N> r) {
+    const long long i = group_id<L>();
+    if (i >= count) return;
+    if (elem_one<N, L, OP, false>(C, x, y, yd, r, i))
+        if constexpr (cold_round(N, L)) elem_rounded<N, OP>(C, x, y, yd, r, i);
 }
 
 // comparisons: r[i] in {-1, 0, 1}. MODE 0: cuda::mp_cmp (src/arith/cmp.cuh:120-124), 1:
@@ -494,48 +490,80 @@ __global__ __launch_bounds__(BLK) void k_soa_to_aos(const DevConsts *__restrict_
 
 // ---------------------------------------------------------------- axpy
 // v1: buffer = x * alpha (+round), y = buffer (+) y with the v1 vector add (+round),
-// src/blas/axpy.cuh:62-72 fused into one pass
+// src/blas/axpy.cuh:62-72 fused into one pass. Bounded by memory traffic while no number needs
+// rounding, by the roundings otherwise; one body serves both (Grp::round_fails). Over 10^6 numbers of
+// 212 (424) bits: 0.063 (0.146) ms with operands that are doubles, before 0.067 (0.145); with full
+// operands 0.26 (0.99) ms, before 2.2 (12.4): their rounding was a mixed-radix evaluation of
+// 16 (32) digits in scratch memory.
+template <int N, int L, bool COLD>
+__device__ __forceinline__ bool axpy_one(const DevConsts *__restrict__ C, const SoA &alpha, const SoA &x, long long ix,
+                                         const SoA &y, long long iy) {
+    Grp<N, L> g(C);
+    MP<N / L> a, xv, yv, r;
+    load_soa(g, a, alpha, 0);
+    load_soa(g, xv, x, ix);
+    load_soa(g, yv, y, iy);
+    g.template mul<false>(r, xv, a);
+    bool full = g.template round_fails<COLD>(r);
+    g.template vadd<false>(r, r, yv);
+    full |= g.template round_fails<COLD>(r);
+    if (full) return g.lane() == 0;
+    store_soa(g, r, y, iy);
+    return false;
+}
+template <int N>
+__device__ __noinline__ void axpy_rounded(const DevConsts *C, SoA alpha, SoA x, long long ix, SoA y, long long iy) {
+    axpy_one<N, 1, true>(uniform_ptr(C), alpha, x, ix, y, iy);
+}
 template <int N, int L>
-__global__ __launch_bounds__(BLK) void k_axpy(const DevConsts *__restrict__ C, int n, SoA alpha, SoA x, int incx, SoA y,
+__global__ __launch_bounds__(BLK) COLD_WAVES(N, L) void k_axpy(const DevConsts *__restrict__ C, int n, SoA alpha, SoA x, int incx, SoA y,
                                               int incy) {
     alpha = rd(alpha);
     x = rd(x);
     y = rd(y);
     const long long i = group_id<L>();
     if (i >= n) return;
-    Grp<N, L> g(C);
-    MP<N / L> a, xv, yv, b, r;
-    load_soa(g, a, alpha, 0);
-    load_soa(g, xv, x, bidx(i, n, incx));
-    const long long iy = bidx(i, n, incy);
-    load_soa(g, yv, y, iy);
-    g.mul(b, xv, a);
-    g.vadd(r, b, yv);
-    store_soa(g, r, y, iy);
+    if (axpy_one<N, L, false>(C, alpha, x, bidx(i, n, incx), y, bidx(i, n, incy)))
+        if constexpr (cold_round(N, L)) axpy_rounded<N>(C, alpha, x, bidx(i, n, incx), y, bidx(i, n, incy));
 }
 // v2: r = alpha * x (+) y, src/blas/v2/axpy_v2.cuh:39-52
 // NEG: mp_maxpy, r = (-alpha) * x (+) y (src/blas/v2/maxpy_v2.cuh)
-template <int N, int L, bool NEG = false>
-__global__ __launch_bounds__(BLK) void k_axpy_v2(const DevConsts *__restrict__ C, int n, AoSRef<N> alpha, AoSRef<N> x,
-                                                 AoSRef<N> y, AoSRef<N> r) {
-    const long long i = group_id<L>();
-    if (i >= n) return;
+template <int N, int L, bool NEG, bool COLD>
+__device__ __forceinline__ bool axpy_v2_one(const DevConsts *__restrict__ C, AoSRef<N> alpha, AoSRef<N> x, AoSRef<N> y,
+                                            AoSRef<N> r, long long i) {
     Grp<N, L> g(C);
-    MP<N / L> a, xv, yv, ax, s;
+    MP<N / L> a, xv, yv, s;
     load_aos(g, a, alpha, 0);
     if (NEG) a.sign ^= 1;
     load_aos(g, xv, x, i);
     load_aos(g, yv, y, i);
-    g.mul(ax, a, xv);
-    g.add(s, ax, yv);
+    g.template mul<false>(s, a, xv);
+    bool full = g.template round_fails<COLD>(s);
+    g.template add<false>(s, s, yv);
+    full |= g.template round_fails<COLD>(s);
+    if (full) return g.lane() == 0;
     store_aos(g, s, r, i);
+    return false;
+}
+template <int N, bool NEG>
+__device__ __noinline__ void axpy_v2_rounded(const DevConsts *C, AoSRef<N> alpha, AoSRef<N> x, AoSRef<N> y, AoSRef<N> r,
+                                             long long i) {
+    axpy_v2_one<N, 1, NEG, true>(uniform_ptr(C), alpha, x, y, r, i);
+}
+template <int N, int L, bool NEG = false>
+__global__ __launch_bounds__(BLK) COLD_WAVES(N, L) void k_axpy_v2(const DevConsts *__restrict__ C, int n, AoSRef<N> alpha, AoSRef<N> x,
+                                                 AoSRef<N> y, AoSRef<N> r) {
+    const long long i = group_id<L>();
+    if (i >= n) return;
+    if (axpy_v2_one<N, L, NEG, false>(C, alpha, x, y, r, i))
+        if constexpr (cold_round(N, L)) axpy_v2_rounded<N, NEG>(C, alpha, x, y, r, i);
 }
 
 // ---------------------------------------------------------------- gemv
 // out[k] = v[k] * s (vec2scal esi/digits/round, src/mpvector.cuh:139-216), v with BLAS stride;
 // out is AoS (ws) or the SoA v itself (in place)
 template <int N, int L, bool INPLACE>
-__global__ __launch_bounds__(BLK) void k_scal(const DevConsts *__restrict__ C, int len, SoA s, SoA v, int inc,
+__global__ __launch_bounds__(BLK) ELEM_WAVES(N, L) void k_scal(const DevConsts *__restrict__ C, int len, SoA s, SoA v, int inc,
                                               AoSRef<N> out) {
     s = rd(s);
     v = rd(v);
@@ -546,7 +574,8 @@ __global__ __launch_bounds__(BLK) void k_scal(const DevConsts *__restrict__ C, i
     load_soa(g, a, s, 0);
     const long long iv = bidx(k, len, inc);
     load_soa(g, x, v, iv);
-    g.mul(r, x, a);
+    g.template mul<false>(r, x, a);
+    g.round_here(r);
     if (INPLACE)
         store_soa(g, r, v, iv);
     else
@@ -583,7 +612,7 @@ __global__ __launch_bounds__(BLK) void k_gemv_fold(const DevConsts *__restrict__
 }
 // y[o] = y[o] (+) rowsum[o]  (src/blas/gemv.cuh:72-75 with mp_add rounding, add.cuh:223-248)
 template <int N, int L>
-__global__ __launch_bounds__(BLK) void k_gemv_final(const DevConsts *__restrict__ C, int len, SoA y, int incy,
+__global__ __launch_bounds__(BLK) ELEM_WAVES(N, L) void k_gemv_final(const DevConsts *__restrict__ C, int len, SoA y, int incy,
                                                     AoSRef<N> sums) {
     y = rd(y);
     const long long o = group_id<L>();
@@ -593,7 +622,8 @@ __global__ __launch_bounds__(BLK) void k_gemv_final(const DevConsts *__restrict_
     const long long iy = bidx(o, len, incy);
     load_soa(g, a, y, iy);
     load_aos(g, s, sums, o);
-    g.add(r, a, s);
+    g.template add<false>(r, a, s);
+    g.round_here(r);
     store_soa(g, r, y, iy);
 }
 
@@ -638,7 +668,7 @@ __global__ __launch_bounds__(BLK) void k_gemm_sum(const DevConsts *__restrict__ 
 //     C = C (+) buffer with the v1 matrix add (+round)
 // v2 (src/blas/v2/gemm_v2.cuh:76-78): C = (sum*alpha) (+) (C*beta)
 template <int N, int L, bool V2, class VM>
-__global__ __launch_bounds__(BLK) void k_gemm_fin(const DevConsts *__restrict__ C_, int m, int n, VM alpha, VM beta,
+__global__ __launch_bounds__(BLK) ELEM_WAVES(N, L) void k_gemm_fin(const DevConsts *__restrict__ C_, int m, int n, VM alpha, VM beta,
                                                   VM Cm, int ldc, AoSRef<N> sums) {
     if constexpr (!V2) {
         alpha = rd(alpha);
@@ -650,7 +680,7 @@ __global__ __launch_bounds__(BLK) void k_gemm_fin(const DevConsts *__restrict__ 
     const int row = (int)(e % m), col = (int)(e / m);
     const long long ic = (long long)col * ldc + row;
     Grp<N, L> g(C_);
-    MP<N / L> sum, a, b, cv, s2, c2, r;
+    MP<N / L> sum, a, b, cv, s2, r;
     load_aos(g, sum, sums, e);
     if constexpr (V2) {
         load_aos(g, a, alpha, 0);
@@ -661,15 +691,19 @@ __global__ __launch_bounds__(BLK) void k_gemm_fin(const DevConsts *__restrict__ 
         load_soa(g, b, beta, 0);
         load_soa(g, cv, Cm, ic);
     }
-    g.mul(s2, sum, a);
-    g.mul(c2, cv, b);
-    if constexpr (V2) {
-        g.add(r, s2, c2);
+    g.template mul<false>(s2, sum, a);
+    g.round_here(s2);
+    g.template mul<false>(r, cv, b);
+    g.round_here(r);
+    if constexpr (V2)
+        g.template add<false>(r, s2, r);
+    else
+        g.template vadd<false>(r, r, s2);
+    g.round_here(r);
+    if constexpr (V2)
         store_aos(g, r, Cm, ic);
-    } else {
-        g.vadd(r, c2, s2);
+    else
         store_soa(g, r, Cm, ic);
-    }
 }
 
 // ---------------------------------------------------------------- gemm, split form

@@ -19,7 +19,7 @@ namespace mph {
 // of V1_MUL is S[0] (SF_SCALAR: vec2scal / mat2scal), S[bidx(i, m, incs)] (SF_ROW:
 // mat2vec_left_scal) or S[bidx(j, n, incs)] (SF_COL: mat2vec_right_scal, cvec2rvec).
 template <int N, int L, int OP, int SF>
-__global__ __launch_bounds__(BLK) void k_v1map(const DevConsts *__restrict__ C, int m, int n, SoA S, int incs, SoA X,
+__global__ __launch_bounds__(BLK) ELEM_WAVES(N, L) void k_v1map(const DevConsts *__restrict__ C, int m, int n, SoA S, int incs, SoA X,
                                                int ldx, int incx, SoA Y, int ldy, int incy, SoA W, int ldw,
                                                int incw) {
     S = rd(S);
@@ -35,12 +35,13 @@ __global__ __launch_bounds__(BLK) void k_v1map(const DevConsts *__restrict__ C, 
     if constexpr (OP == V1_MUL) {
         const long long is = SF == SF_SCALAR ? 0 : (SF == SF_ROW ? bidx(i, m, incs) : bidx(j, n, incs));
         load_soa(g, b, S, is);
-        g.mul(r, a, b);
+        g.template mul<false>(r, a, b);
     } else {
         load_soa(g, b, Y, bidx(i, m, incy) + (long long)j * ldy);
         if (OP == V1_SUB) b.sign ^= 1;
-        g.vadd(r, a, b);
+        g.template vadd<false>(r, a, b);
     }
+    g.round_here(r);
     store_soa(g, r, W, bidx(i, m, incw) + (long long)j * ldw);
 }
 

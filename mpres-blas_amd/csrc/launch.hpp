@@ -82,7 +82,7 @@ struct Launch {
         return hipGetLastError();
     }
     // pass 0: the main kernel; pass 1: the fixup kernel over the chains marked
-    static constexpr bool SPLIT = !Grp<N, L>::INL;
+    static constexpr bool SPLIT = N > 8;
     template <int MODE>
     static void fold_pass(int pass, const dim3 &gr, const DevConsts *c, long long cnt, long long nvt, SoA xs, int incx,
                           SoA ys, int incy, AoSRef<N> XA, AoSRef<N> YA, AoSRef<N> O, hipStream_t st) {

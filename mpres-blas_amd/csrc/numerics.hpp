@@ -370,6 +370,32 @@ MPH_HD int mulmod(int a, int b, double m, double minv) {
     double r = fma(-q, m, p) + pl;
     return (int)mod_fix1(r, m);
 }
+// (a * w) mod m for a fixed factor w < m < 2^31 with wq = floor(w 2^32 / m) (mulmod_q) and any a < 2^32:
+// q = floor(a wq / 2^32) is the quotient or one less, so a w - q m (mod 2^32) lies in [0, 2m). Six
+// integer instructions, all full rate, against about eighteen of mulmod.
+MPH_HD int mulmod_c(uint32_t a, uint32_t w, uint32_t wq, uint32_t m) {
+    const uint32_t q = (uint32_t)(((uint64_t)a * wq) >> 32);
+    const uint32_t r = a * w - q * m, s = r - m;
+    return (int)(r < s ? r : s);
+}
+// (a * b) mod m for 0 <= a, b < m, 2^s <= m < 1.43e9 (so 3 m < 2^32, s <= 30), mu = floor(2^(s + 32) / m):
+// q = floor(floor(a b / 2^s) mu / 2^32) is the quotient, or up to two less (the first floor costs
+// less than 2^s / m <= 1, mu's less than a b / 2^(s + 32) <= 1), so a b - q m (mod 2^32) lies in
+// [0, 3m). Nine integer instructions, all full rate, where mulmod takes about eighteen.
+MPH_HD int mulmod_i(uint32_t a, uint32_t b, uint32_t m, uint32_t mu, int s) {
+    const uint64_t p = (uint64_t)a * b;
+#if defined(__HIP_DEVICE_COMPILE__)
+    const uint32_t h = __builtin_amdgcn_alignbit((uint32_t)(p >> 32), (uint32_t)p, (uint32_t)s);
+#else
+    const uint32_t h = (uint32_t)(p >> s);
+#endif
+    const uint32_t q = (uint32_t)(((uint64_t)h * mu) >> 32);
+    uint32_t r = (uint32_t)p - q * m;
+    uint32_t t = r - m;
+    r = r < t ? r : t;
+    t = r - m;
+    return (int)(r < t ? r : t);
+}
 // v mod m for an integer-valued 0 <= v < 2^53 (q is again within one of v / m)
 MPH_HD int modd(double v, double m, double minv) {
     const double q = floor(v * minv);

@@ -22,17 +22,10 @@
 // that cancel exactly to zero are left to the residue kernels.
 #pragma once
 
-#include <type_traits>
-
 #include "bigint.hpp"
 #include "group.hpp"
 
 namespace mph {
-
-template <int N>
-struct Pos {
-    static constexpr int W = N / 2;  // words of a normalised number (at most 31 N / 2 + 2 bits)
-};
 
 // an operand of a product
 template <int W>
@@ -72,24 +65,6 @@ constexpr double POS_FRESH = 0x1p-22;  // relative distance of a computed evalua
 constexpr double POS_GIVEN = 0x1p-20;  // of an operand's
 constexpr double POS_PROD = 0x1.01p-19;  // of a product of two such operands
 
-// a value of the constants block, through the scalar cache: the address is wave-uniform and the
-// block is never written while kernels run, which the constant address space states (a plain
-// load behind calls and stores would be a vector load)
-template <class T>
-__device__ __forceinline__ T pos_const(const T &v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    return *(const __attribute__((address_space(4))) T *)(uintptr_t)&v;
-#else
-    return v;
-#endif
-}
-// keeps the instructions before it ahead of those after it: bounds how many table entries are
-// in registers at once
-__device__ __forceinline__ void pos_fence() {
-#if defined(__HIP_DEVICE_COMPILE__)
-    __builtin_amdgcn_sched_barrier(0);
-#endif
-}
 __device__ __forceinline__ int pos_ilogb(double v) {  // floor(log2 v), v > 0 normal
 #if defined(__HIP_DEVICE_COMPILE__)
     return __builtin_amdgcn_frexp_exp(v) - 1;
@@ -105,32 +80,6 @@ __device__ __forceinline__ double pos_double(const uint32_t *x) {
 #pragma unroll
     for (int i = W - 2; i >= 0; i--) h = fma(h, 0x1p32, (double)x[i]);
     return h;
-}
-// x >> s for any s >= 0; dropped: whether a nonzero bit was shifted out
-template <int W>
-__device__ __forceinline__ void pos_shr(uint32_t *r, const uint32_t *x, int s, bool &dropped) {
-    uint32_t low = 0;
-    const int b = s & 31;
-    int q = s >> 5;
-    q = q > W ? W : q;
-#pragma unroll
-    for (int i = 0; i < W; i++) r[i] = x[i];
-#pragma unroll
-    for (int k = 1; k <= W; k <<= 1) {
-        const bool on = (q & k) != 0;
-#pragma unroll
-        for (int i = 0; i < W; i++) {
-            if (i < k) low |= on ? r[i] : 0u;
-            r[i] = on ? (i + k < W ? r[i + k] : 0u) : r[i];
-        }
-    }
-    low |= b ? r[0] << ((32 - b) & 31) : 0u;
-#pragma unroll
-    for (int i = 0; i < W; i++) {
-        const uint32_t hi = i + 1 < W ? r[i + 1] : 0u;
-        r[i] = (uint32_t)((((uint64_t)hi << 32) | r[i]) >> b);
-    }
-    dropped = low != 0;
 }
 // x << s, s >= 0, the result below 2^(32 W)
 template <int W>
@@ -151,147 +100,6 @@ __device__ __forceinline__ void pos_shl(uint32_t *r, const uint32_t *x, int s) {
     }
 }
 
-// the integer of normalised residues (X / M below 2^-40): X = sum c_i M/m_i - rank M with
-// c_i = |x_i w_i| mod m_i. rank is the nearest integer of sum c_i / m_i. Sums run over 16-bit
-// limbs of the constants in doubles: 32 products below 2^47 and a carry stay below 2^53.
-template <int N>
-__device__ __forceinline__ void pos_from_digits(const DevConsts *__restrict__ C, const int *d, uint32_t *x) {
-    constexpr int W = Pos<N>::W;
-    double c[N], rk = 0.0;
-#pragma unroll
-    for (int i = 0; i < N; i++) {
-        c[i] = (double)mulmod(d[i], pos_const(C->w[i]), pos_const(C->md[i]), pos_const(C->minv[i]));
-        rk = fma(c[i], pos_const(C->minv[i]), rk);
-    }
-    rk = rint(rk);
-    double carry = 0.0;
-#pragma unroll
-    for (int l = 0; l < W; l++) {
-        uint32_t half[2];
-        pos_fence();
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            double v = carry;
-#pragma unroll
-            for (int i = 0; i < N; i++) v = fma(c[i], pos_const(C->mi16[2 * l + u][i]), v);
-            v = fma(-rk, pos_const(C->m16[2 * l + u]), v);
-            carry = floor(v * 0x1p-16);
-            half[u] = (uint32_t)fma(carry, -0x1p16, v);
-        }
-        x[l] = half[0] | (half[1] << 16);
-    }
-}
-// residue i of an integer of WX words
-template <int N, int WX>
-__device__ __forceinline__ int pos_residue(const DevConsts *__restrict__ C, const uint32_t *x, int i) {
-    double v = 0.0;
-#pragma unroll
-    for (int l = 0; l < WX; l++) {
-        v = fma((double)(x[l] & 0xffffu), pos_const(C->q16[2 * l][i]), v);
-        v = fma((double)(x[l] >> 16), pos_const(C->q16[2 * l + 1][i]), v);
-    }
-    return modd(v, pos_const(C->md[i]), pos_const(C->minv[i]));
-}
-// ---- several directed operations under one setting of the rounding mode (numerics.hpp) ----
-#if defined(__HIP_DEVICE_COMPILE__)
-#define POS_DIR4(MODE, OP)                                                                                \
-    asm("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), " #MODE "\n\ts_nop 1\n\t" OP " %0, %4, %5\n\t" OP  \
-        " %1, %6, %7\n\t" OP " %2, %8, %9\n\t" OP " %3, %10, %11\n\ts_nop 1\n\t"                         \
-        "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 0\n\ts_nop 1"                                       \
-        : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3])                                              \
-        : "v"(a[0]), "v"(b[0]), "v"(a[1]), "v"(b[1]), "v"(a[2]), "v"(b[2]), "v"(a[3]), "v"(b[3]))
-#endif
-// r[i] = a[i] * b[i] (MUL) or a[i] + b[i] rounded up (UP) or down, i < CNT
-template <int CNT, bool MUL, bool UP>
-__device__ __forceinline__ void dir_n(double *r, const double *a, const double *b) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    if constexpr (CNT >= 4) {
-        if constexpr (MUL && UP) POS_DIR4(1, "v_mul_f64");
-        if constexpr (MUL && !UP) POS_DIR4(2, "v_mul_f64");
-        if constexpr (!MUL && UP) POS_DIR4(1, "v_add_f64");
-        if constexpr (!MUL && !UP) POS_DIR4(2, "v_add_f64");
-        if constexpr (CNT > 4) dir_n<CNT - 4, MUL, UP>(r + 4, a + 4, b + 4);
-        return;
-    }
-#endif
-#pragma unroll
-    for (int i = 0; i < CNT; i++) r[i] = MUL ? (UP ? mul_ru(a[i], b[i]) : mul_rd(a[i], b[i]))
-                                             : (UP ? add_ru(a[i], b[i]) : add_rd(a[i], b[i]));
-}
-#undef POS_DIR4
-// psum_arr's balanced tree over v[0 .. CNT-1], in place; the sum in v[0]
-template <int CNT, bool UP>
-__device__ __forceinline__ void dir_sum(double *v) {
-    if constexpr (CNT > 1) {
-        double a[CNT / 2], b[CNT / 2];
-#pragma unroll
-        for (int i = 0; i < CNT / 2; i++) {
-            a[i] = v[2 * i];
-            b[i] = v[2 * i + 1];
-        }
-        dir_n<CNT / 2, false, UP>(v, a, b);
-        dir_sum<CNT / 2, UP>(v);
-    }
-}
-// Interval evaluation of a rounded integer: rns_eval<FULL = false> on its residues, the
-// directed operations of one kind issued together.
-template <int N>
-__device__ __forceinline__ void pos_eval_fast(const DevConsts *__restrict__ C, const uint32_t *x, Er &lo, Er &up) {
-    int s[N];
-    double a[N], rc[N], f[N];
-#pragma unroll
-    for (int i = 0; i < N; i++) {
-        s[i] = mulmod(pos_residue<N, Pos<N>::W>(C, x, i), pos_const(C->w[i]), pos_const(C->md[i]),
-                      pos_const(C->minv[i]));
-        pos_fence();
-    }
-    auto sum = [&](auto upw, double &frac, unsigned &whole) {
-        constexpr bool UP = decltype(upw)::value;
-#pragma unroll
-        for (int i = 0; i < N; i++) {
-            a[i] = (double)s[i];
-            rc[i] = UP ? pos_const(C->rru[i]) : pos_const(C->rrd[i]);
-        }
-        dir_n<N, true, UP>(f, a, rc);
-        dir_sum<N, UP>(f);
-        whole = (unsigned)f[0];
-        frac = f[0];
-    };
-    double sl, su;
-    unsigned wl, wu;
-    sum(std::false_type{}, sl, wl);
-    sum(std::true_type{}, su, wu);
-    if (sl == 0 && su == 0) {
-        lo = Er{0.0, 0};
-        up = Er{0.0, 0};
-        return;
-    }
-    sl = sub_rd(sl, (double)wl);
-    su = sub_ru(su, (double)wu);
-    const double acc = pos_const(C->acc);
-    int K = 0;
-    if (su < acc) {
-        const int ref = pos_const(C->ref_factor), kmax = pos_const(C->log2m);
-        const int *p2 = pos_const(C->pow2);
-        for (int it = 0; su < acc && it < EVAL_MAX_ITER; it++) {
-            int kk = -(ceil_log2_rn(su) + 1);
-            kk = kk > ref ? kk : ref;
-            kk = kk < kmax ? kk : kmax;
-            const int *row = p2 + (size_t)kk * N;
-#pragma unroll
-            for (int i = 0; i < N; i++) s[i] = mulmod(s[i], row[i], pos_const(C->md[i]), pos_const(C->minv[i]));
-            sum(std::true_type{}, su, wu);
-            su = sub_ru(su, (double)wu);
-            K += kk;
-        }
-        sum(std::false_type{}, sl, wl);
-        sl = sub_rd(sl, (double)wl);
-    }
-    lo = er_set_d(sl);
-    up = er_set_d(su);
-    lo.exp -= K;
-    up.exp -= K;
-}
 // the same; U: in registers (the end of a chain), or with rolled loops, for the rare
 // out-of-line calls
 template <int N, bool U>
@@ -312,7 +120,7 @@ template <int N>
 __device__ __forceinline__ void pos_operand(const DevConsts *__restrict__ C, const int *d, int s, int e, Er e0, Er e1,
                                             PosOp<Pos<N>::W> &o) {
     constexpr int W = Pos<N>::W;
-    pos_from_digits<N>(C, d, o.x);
+    pos_from_digits<N, W, true>(C, d, o.x);
     o.e = e;
     o.s = s;
     o.h = pos_double<W>(o.x);

@@ -22,16 +22,17 @@ namespace mph {
 template <int N, int L>
 struct Core {
     static constexpr int R = N / L;
-    // One residue per lane on the inlined paths (8 moduli on 8 lanes, where rounding runs on
-    // almost every step): the lane's constants are read once, by load(), and held in
+    // One residue per lane (the inlined paths; at 8 moduli rounding runs on almost every step):
+    // the lane's constants are read once, by load(), and held in
     // registers, so that no step waits on a reload of them. Otherwise they are read where used.
-    static constexpr bool KC = (N <= 8 && R == 1);
+    static constexpr bool KC = (R == 1);
     static constexpr int KN = KC ? N - 1 : 1;
     const DevConsts *__restrict__ C;
     const int *__restrict__ P2;
     int lane;
     double kmd, kmv, krd, kru;
     int kmi, kw, kmrc[KN];
+    uint32_t kwq;
     __device__ __forceinline__ void load() {
         if constexpr (KC) {
             kmd = C->md[lane];
@@ -40,6 +41,7 @@ struct Core {
             kru = C->rru[lane];
             kmi = C->m[lane];
             kw = C->w[lane];
+            kwq = C->wq[lane];
 #pragma unroll
             for (int j = 0; j < KN; j++) kmrc[j] = C->mrcinv[j][lane];
         }
@@ -60,6 +62,19 @@ struct Core {
     __device__ __forceinline__ int w(int r) const {
         if constexpr (KC) return kw;
         else return C->w[ix(r)];
+    }
+    __device__ __forceinline__ uint32_t wq(int r) const {
+        if constexpr (KC) return kwq;
+        else return C->wq[ix(r)];
+    }
+    // x_r times the weight w_r, mod m_r
+    __device__ __forceinline__ int xw(int x, int r) const {
+        return mulmod_c((uint32_t)x, (uint32_t)w(r), wq(r), (uint32_t)mi(r));
+    }
+    // x times RNS_POW2's entry at row k for residue r, mod m_r
+    __device__ __forceinline__ int xpow2(int x, int k, int r, uint32_t m) const {
+        const int *p = P2 + (size_t)k * N + ix(r);
+        return mulmod_c((uint32_t)x, (uint32_t)p[0], (uint32_t)p[(size_t)(C->log2m + 1) * N], m);
     }
     __device__ __forceinline__ double rrd(int r) const {
         if constexpr (KC) return krd;
@@ -221,7 +236,7 @@ __device__ __forceinline__ void rns_eval(Core<N, L> k, const int *x, Er &lo, Er 
     int s[R];
     double fl[R], fu[R];
     loop<R, U>([&](int r) {
-        s[r] = mulmod(x[r], k.w(r), k.md(r), k.mv(r));
+        s[r] = k.xw(x[r], r);
         fl[r] = mul_rd((double)s[r], k.rrd(r));
         fu[r] = mul_ru((double)s[r], k.rru(r));
     });
@@ -260,9 +275,8 @@ __device__ __forceinline__ void rns_eval(Core<N, L> k, const int *x, Er &lo, Er 
         int kk = -(ceil_log2_rn(sumu) + 1);
         kk = kk > ref ? kk : ref;
         kk = kk < kmax ? kk : kmax;
-        const int *row = k.P2 + (size_t)kk * N;
         loop<R, U>([&](int r) {
-            s[r] = mulmod(s[r], row[k.ix(r)], k.md(r), k.mv(r));
+            s[r] = k.xpow2(s[r], kk, r, (uint32_t)k.mi(r));
             fu[r] = mul_ru((double)s[r], k.rru(r));
         });
         sumu = psum_arr<N, L, true, U>(fu);
@@ -311,13 +325,14 @@ __device__ __forceinline__ void rns_scale_step(Core<N, L> k, int *y, int kr, int
         const int mult = modd((double)res, k.md(r), k.mv(r));
         int t = x[r] - mult;
         t = t < 0 ? t + k.mi(r) : t;
-        y[r] = mulmod(t, k.C->pow2inv[j - 1][k.ix(r)], k.md(r), k.mv(r));
+        y[r] = mulmod_c((uint32_t)t, (uint32_t)k.C->pow2inv[j - 1][k.ix(r)], k.C->pow2invq[j - 1][k.ix(r)],
+                        (uint32_t)k.mi(r));
     });
 }
 template <int N, int L, bool U>
 __device__ __forceinline__ void rns_xw(Core<N, L> k, int *c, const int *x) {
     constexpr int R = N / L;
-    loop<R, U>([&](int r) { c[r] = mulmod(x[r], k.w(r), k.md(r), k.mv(r)); });
+    loop<R, U>([&](int r) { c[r] = k.xw(x[r], r); });
 }
 template <int N, int L, bool U>
 __device__ __forceinline__ void rns_scale2pow(Core<N, L> k, int *x, unsigned D) {
@@ -354,7 +369,7 @@ __device__ __forceinline__ void mp_round_body(Core<N, L> k, int *d, int &exp, Er
 }
 
 // ---------------- out-of-line entry points (U = false) ----------------
-template <int N, int L>
+template <int N, int L, bool ELEM = false>  // ELEM: the element kernels' copy (Grp::round_here)
 __device__ __noinline__ void ool_round(Core<N, L> k, int *d, int *exp, Er *ev0, Er *ev1) {
     int e = *exp;
     Er a = *ev0, b = *ev1;

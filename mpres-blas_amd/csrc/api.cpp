@@ -1257,17 +1257,34 @@ struct mpres_batch {
 
 namespace {
 
-int batch_resolve(const mpres_ctx *c, const mpres_batch_tuning_t *t, mpres_batch_tuning_t &u, const Ops **ops) {
-    // built-in geometry: the autotuner's best on the batching workload at 16 moduli
-    // (mpres-blas_amd/tuning/batch_gfx950.json): the gemv lanes (4 at 16 moduli), 4
-    // workgroups per CU, 128 gemv rows per item
-    u.lanes = (t && t->lanes) ? t->lanes : c->ops[OP_GEMV]->L;
+// Lanes of a batch, where the caller leaves them to the plan. Over 16 moduli, one lane a number
+// (its roundings positional) if the costliest problem is a gemv with more chains than a workgroup has
+// lanes, the gemv lanes (4) otherwise: 1024 dots and gemvs of 32 to 1024 rows in 12.0 ms with
+// one lane and 23.7 with 4 (half as far spread operands, which round seldom: 6.5 and 7.7 ms); 512
+// dots of 16 x 64 chains 0.42 and 0.36 ms.
+int batch_lanes(const mpres_ctx *c, const mpres_batch_problem_t *probs, int count) {
+    const int L = c->ops[OP_GEMV]->L;
+    int i;
+    if (c->host.n != 16 || !c->lt[OP_GEMV].builtin || batch_fmas(probs, count, i) <= 0) return L;
+    const mpres_batch_problem_t &p = probs[i];
+    if (p.op != MPRES_BATCH_GEMV) return L;
+    const int ly = p.trans == MPRES_NO_TRANS ? p.m : p.n;
+    return (double)ly * p.block3 > 256 ? 1 : L;
+}
+
+// groups: for batch_layout, 0 where the caller gave the rows per item
+int batch_resolve(const mpres_ctx *c, const mpres_batch_problem_t *probs, int count, const mpres_batch_tuning_t *t,
+                  mpres_batch_tuning_t &u, const Ops **ops, int &groups) {
+    // built-in geometry: batch_lanes, 4 workgroups per CU, and up to 128 gemv rows per item
+    // (batch_rows; mpres-blas_amd/tuning/batch_gfx950.json holds the sweep with rows fixed)
+    u.lanes = (t && t->lanes) ? t->lanes : batch_lanes(c, probs, count);
     u.wg_per_cu = (t && t->wg_per_cu) ? t->wg_per_cu : 4;
     u.gemv_rows = (t && t->gemv_rows) ? t->gemv_rows : 128;
     if (u.wg_per_cu < 0 || u.wg_per_cu > 32 || u.gemv_rows < 0)
         return fail(MPRES_ERR_ARG, "invalid batch tuning (%d workgroups per CU, %d rows)", u.wg_per_cu, u.gemv_rows);
     *ops = find_ops(c->host.n, u.lanes);
     if (!*ops) return fail(MPRES_ERR_UNSUPPORTED, "%d lanes per number not compiled for %d moduli", u.lanes, c->host.n);
+    groups = (t && t->gemv_rows) ? 0 : 256 / u.lanes;
     return MPRES_OK;
 }
 
@@ -1288,9 +1305,10 @@ size_t mpres_batch_workspace(const mpres_ctx_t *c, const mpres_batch_problem_t *
     if (!c) return 0;
     mpres_batch_tuning_t u;
     const Ops *o;
-    if (batch_resolve(c, tuning, u, &o)) return 0;
+    int groups;
+    if (batch_resolve(c, probs, count, tuning, u, &o, groups)) return 0;
     BatchLayout lay;
-    if (batch_layout(probs, count, c->host.n, u.gemv_rows, lay)) return 0;
+    if (batch_layout(probs, count, c->host.n, u.gemv_rows, lay, groups)) return 0;
     return lay.ws_bytes;
 }
 
@@ -1300,10 +1318,13 @@ int mpres_batch_plan(mpres_ctx_t *c, const mpres_batch_problem_t *probs, int cou
     *plan = nullptr;
     mpres_batch_tuning_t u;
     const Ops *o;
-    int rc = batch_resolve(c, tuning, u, &o);
+    int groups;
+    int rc = batch_resolve(c, probs, count, tuning, u, &o, groups);
     if (rc) return rc;
     BatchLayout lay;
-    rc = batch_layout(probs, count, c->host.n, u.gemv_rows, lay);
+    rc = batch_layout(probs, count, c->host.n, u.gemv_rows, lay, groups);
+    if (!rc && ws && groups && wsb < lay.ws_bytes)  // a workspace for fewer, larger items
+        rc = batch_layout(probs, count, c->host.n, u.gemv_rows, lay);
     if (rc) return fail(rc, "%s", lay.err.c_str());
     if (ws && wsb < lay.ws_bytes)
         return fail(MPRES_ERR_WORKSPACE, "workspace of %zu bytes, %zu needed", wsb, lay.ws_bytes);

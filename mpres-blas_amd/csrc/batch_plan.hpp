@@ -4,6 +4,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <string>
 #include <vector>
@@ -33,10 +34,44 @@ struct BatchLayout {
 
 constexpr size_t BATCH_WS_ALIGN = 256;
 
+// Rows per item of a gemv of ly outputs, lx terms each, in block3 chains, where the plan chooses them
+// (at most cap): an item is to be no more than 1 / BATCH_PARTS of the batch's multiply-accumulates,
+// so that its slowest item does not outlast the others (about two items a compute unit), but gives each
+// group of lanes of its workgroup (groups) a chain; the rows are split evenly. Every item forms
+// alpha * x again, which costs it lx products beside rows * lx. One gemv of 1024^2 over 16 moduli,
+// before in items of 128 rows: 17.2 -> 2.2 ms; 512 gemvs of 48 rows keep one item each (0.26 ms;
+// two each 0.34).
+constexpr int BATCH_PARTS = 512;
+inline int batch_rows(double fmas, int lx, int ly, int block3, int groups, int cap) {
+    const double fair = std::ceil(fmas / BATCH_PARTS / lx);
+    const int least = std::max(1, (groups + block3 - 1) / block3);
+    int rows = fair < cap ? std::max((int)fair, least) : cap;
+    rows = std::min(rows, cap);
+    const int parts = (ly + rows - 1) / rows;
+    return (ly + parts - 1) / parts;
+}
+// multiply-accumulates of a batch; costliest: index of the problem with the most (-1: none)
+inline double batch_fmas(const mpres_batch_problem_t *probs, int count, int &costliest) {
+    double sum = 0, most = 0;
+    costliest = -1;
+    for (int i = 0; probs && i < count; i++) {
+        const mpres_batch_problem_t &p = probs[i];
+        const double f = p.op == MPRES_BATCH_DOT ? (p.n > 0 ? p.n : 0)
+                                                 : (p.m > 0 && p.n > 0 ? (double)p.m * p.n : 0);
+        sum += f;
+        if (f > most) {
+            most = f;
+            costliest = i;
+        }
+    }
+    return sum;
+}
+
 // Returns MPRES_OK, or MPRES_ERR_ARG with layout.err naming the first bad problem.
 // Problems the single call would skip (dot n <= 0, gemv m or n <= 0) give no item.
+// groups > 0: gemv_rows is the most that batch_rows may choose, for workgroups of that many groups
 inline int batch_layout(const mpres_batch_problem_t *probs, int count, int n_moduli, int gemv_rows,
-                        BatchLayout &out) {
+                        BatchLayout &out, int groups = 0) {
     out = BatchLayout{};
     const long long S = 4LL * n_moduli + 40;
     char buf[160];
@@ -59,6 +94,8 @@ inline int batch_layout(const mpres_batch_problem_t *probs, int count, int n_mod
         size_t bytes;
     };
     std::vector<Work> v;
+    int costliest;
+    const double total = batch_fmas(probs, count, costliest);
     for (int i = 0; i < count; i++) {
         const mpres_batch_problem_t &p = probs[i];
         if (p.op == MPRES_BATCH_DOT) {
@@ -93,8 +130,9 @@ inline int batch_layout(const mpres_batch_problem_t *probs, int count, int n_mod
             const bool tr = p.trans != MPRES_NO_TRANS;
             const int lx = tr ? p.m : p.n, ly = tr ? p.n : p.m;
             out.fmas += (double)p.m * p.n;
-            for (int r0 = 0; r0 < ly; r0 += gemv_rows) {
-                const int r1 = std::min(ly, r0 + gemv_rows), h = r1 - r0;
+            const int rows = groups > 0 ? batch_rows(total, lx, ly, p.block3, groups, gemv_rows) : gemv_rows;
+            for (int r0 = 0; r0 < ly; r0 += rows) {
+                const int r1 = ly - r0 > rows ? r0 + rows : ly, h = r1 - r0;
                 Work w{};
                 w.it.kind = tr ? BATCH_GEMV_T : BATCH_GEMV_N;
                 w.it.r0 = r0;

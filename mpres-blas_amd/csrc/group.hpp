@@ -193,7 +193,8 @@ __device__ __forceinline__ bool sc_fma_step(const ScC &C, Sc &acc, int xs, int x
 
 // the rounding of a number held by one lane, out of line (rare at 16 and 32 moduli)
 template <int N>
-__device__ __noinline__ void ool_pos_round(const DevConsts *C, int *d, int *exp, Er *ev0, Er *ev1) {
+__device__ __noinline__ void ool_pos_round(const DevConsts *C0, int *d, int *exp, Er *ev0, Er *ev1) {
+    const DevConsts *C = uniform_ptr(C0);
     int e = *exp, t[N];
     Er a = *ev0, b = *ev1;
 #pragma unroll

@@ -60,6 +60,24 @@ long long emu_batch_workspace(int set_id, const mpres_batch_problem_t *probs, in
     return rc ? rc : (long long)lay.ws_bytes;
 }
 
+// items where the plan chooses the rows (at most cap, groups of lanes per workgroup): for each, its
+// kind, rows and columns, row range, and scratch range; returns the item count
+int emu_batch_auto(int set_id, const mpres_batch_problem_t *probs, int count, int rows, int groups, long long *out,
+                   int cap, long long *ws_bytes) {
+    const ModuliSet *s = get_set(set_id);
+    if (!s) return -1;
+    BatchLayout lay;
+    const int rc = batch_layout(probs, count, s->n, rows, lay, groups);
+    if (rc) return rc;
+    for (int i = 0; i < (int)lay.items.size() && i < cap; i++) {
+        const BatchItem &t = lay.items[i];
+        const long long v[6] = {t.kind, t.m, t.n, t.r0, t.r1, t.ws};
+        for (int q = 0; q < 6; q++) out[6 * i + q] = v[q];
+    }
+    *ws_bytes = (long long)lay.ws_bytes;
+    return (int)lay.items.size();
+}
+
 // item kinds, row ranges and scratch offsets in launch order (up to cap items); returns the item count
 int emu_batch_items(int set_id, const mpres_batch_problem_t *probs, int count, int rows, int *kind, int *r0, int *r1,
                     long long *off, int cap) {

@@ -167,3 +167,38 @@ def test_batch_rejects_bad_problems(bemu):
         arr = (mp.BatchProblem * 1)(p)
         assert bemu.emu_batch_workspace(sid, arr, 1, 16) == -1
     assert bemu.emu_batch_workspace(sid, (mp.BatchProblem * 1)(bad[0]), 1, 0) == -1
+
+
+@pytest.mark.parametrize("sizes,block3,groups", [([1024], 8, 256), ([1, 31, 33, 700], 8, 256), ([48] * 512, 8, 256),
+                                                 ([5, 1000], 64, 256), ([300, 17, 999], 3, 64), ([2000], 1, 32)])
+@pytest.mark.parametrize("trans", [mp.NO_TRANS, mp.TRANS])
+def test_batch_rows_chosen(bemu, sizes, block3, groups, trans):
+    """rows per item chosen by the plan: every output once, no item above the cap, runs of even
+    length, a chain for every group where the rows allow it, items no larger than the batch's share
+    unless that rule or the cap's holds, scratch ranges disjoint"""
+    o = po.Oracle("16_4double")
+    sid = po.set_names().index("16_4double")
+    x = HostArray(o, o.set_d(gen.uexp(1, 4, -3, 3), D))  # layout reads no numbers
+    p = C.addressof(x.s)
+    arr = (mp.BatchProblem * len(sizes))(*[mp.BatchProblem(
+        op=mp.BATCH_GEMV, trans=trans, m=z, n=z + 2 * i, lda=z, incx=1, incy=1, block3=block3, alpha=p, A=p, x=p, beta=p,
+        y=p) for i, z in enumerate(sizes)])
+    cap, out, wsb = 20000, np.zeros((20000, 6), np.int64), C.c_longlong()
+    cnt = bemu.emu_batch_auto(sid, arr, len(sizes), 128, groups, out.ctypes.data_as(C.c_void_p), cap, C.byref(wsb))
+    it = out[:cnt]
+    total = sum(z * (z + 2 * i) for i, z in enumerate(sizes))
+    for i, z in enumerate(sizes):
+        n = z + 2 * i
+        ly, lx = (z, n) if trans == mp.NO_TRANS else (n, z)
+        runs = sorted((int(a), int(b)) for _, m_, n_, a, b, _ in it if (m_, n_) == (z, n))
+        assert len(runs) % sum((q, q + 2 * j) == (z, n) for j, q in enumerate(sizes)) == 0
+        runs = sorted(set(runs))
+        assert runs[0][0] == 0 and runs[-1][1] == ly
+        assert all(a[1] == b[0] for a, b in zip(runs, runs[1:]))
+        h = [b - a for a, b in runs]
+        assert max(h) <= 128 and len(set(h[:-1])) <= 1 and h[-1] <= h[0]
+        least = -(-groups // block3)
+        assert (max(h) - 1) * lx <= total / 512 or max(h) <= least
+    S = 4 * 16 + 40
+    spans = sorted((int(w), int(w) + ((n_ if trans == mp.NO_TRANS else m_) + (b - a) * block3) * S) for _, m_, n_, a, b, w in it)
+    assert all(a[1] <= b[0] for a, b in zip(spans, spans[1:])) and spans[-1][1] <= wsb.value

@@ -412,9 +412,8 @@ __device__ __forceinline__ void mf_exact_sum(const Grp<N, 1> &g, const DevConsts
     }
     BigN<N> Mb;
     big_zero(Mb);
-    Mb.l[0] = 1u;
 #pragma unroll
-    for (int i = 0; i < N; i++) big_mul_add_u32(Mb, (uint32_t)C_->m[i], 0u);
+    for (int i = 0; i < N; i++) Mb.l[i] = pos_const(C_->m32[i]);
     const BigN<N> Xa = residues_to_big<N>(C_, a.d);
 #pragma unroll 1
     for (int t = 0; t < 4; t++) {
@@ -456,21 +455,27 @@ __device__ __forceinline__ void mf_exact_sum(const Grp<N, 1> &g, const DevConsts
     const int tz = big_ctz(A);
     A = big_shr(A, tz);
     exp += tz;
-    // the rounded significand has at most MP_PRECISION + 1 < log2 M bits: WX limbs hold it
-    BigN<N> R;
+    // The rounded significand has at most MP_PRECISION + 1 bits: Pos<N>::W words hold it. So far
+    // below M the full evaluation is pos_eval_fast's, as in Grp::set_d.
+    uint32_t x[Pos<N>::W];
 #pragma unroll
-    for (int i = 0; i < WX; i++) R.l[i] = A.l[i];
+    for (int i = 0; i < Pos<N>::W; i++) x[i] = A.l[i];
 #pragma unroll
-    for (int i = 0; i < N; i++) res.d[i] = big_mod_d(R, C_->md[i], C_->minv[i]);
+    for (int i = 0; i < N; i++) res.d[i] = pos_residue<N, Pos<N>::W>(C_, x, i);
     res.sign = sign;
     res.exp = exp;
-    g.eval_full(res.d, res.ev0, res.ev1);
+    pos_eval_fast<N>(C_, x, res.ev0, res.ev1);
 }
 
 // The finish at 8 moduli with one rounding per entry: alpha * (the exact band-pair sums)
 // + beta * C is formed exactly in integers (one thread per entry) and rounded once to
 // MP_PRECISION bits, to nearest (ties to even); the result is that significand without
 // trailing zeros, its residues and the full interval evaluation.
+// Bounded by its integer instructions, about 5500 a wave where one pair of bands is live (two CRTs
+// for alpha and beta, one for C, one a pair, products and shifts of up to MF_XS limbs); 2048 x 2048
+// entries in 0.65 ms. Taking the significand's residues and evaluation from its words (pos_residue,
+// pos_eval_fast) in place of divisions and the evaluation of residues, with M's words from the
+// constants, took it from 1.01 ms.
 constexpr int MF_XS = 24, MF_XW = 48;  // 32-bit limbs of the exact accumulation (common, widest)
 
 // One entry's terms: alpha, beta and C loaded, the live terms (bit t: band pair t, then

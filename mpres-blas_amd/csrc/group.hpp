@@ -212,6 +212,16 @@ __device__ __noinline__ void ool_pos_round(const DevConsts *C0, int *d, int *exp
     *ev1 = b;
 }
 
+// residues r0 .. r0 + count - 1 of one lane's numbers x and y (y may be null), any ints, to [0, m)
+__device__ __noinline__ void ool_reduce(const DevConsts *C, int *x, int *y, int r0, int count) {
+#pragma nounroll
+    for (int r = 0; r < count; r++) {
+        const double md = C->md[r0 + r], mv = C->minv[r0 + r];
+        x[r] = modd((double)x[r], md, mv);
+        if (y) y[r] = modd((double)y[r], md, mv);
+    }
+}
+
 // element kernels that round in a function of their own (Grp::round_fails). With more lanes a
 // number that function, run by one lane of the group, leaves the others idle: over 32 moduli and
 // 10^6 full products 8 lanes took 3.5 ms with it, one lane 0.66
@@ -293,6 +303,69 @@ struct Grp {
     }
     __device__ __forceinline__ int mmul(int a, int b, int r, const DevConsts *c) const {
         return mulmod_i((uint32_t)a, (uint32_t)b, (uint32_t)mi(r, c), mu(r, c), mus);
+    }
+    // Residues as a number is stored. Every operation leaves them in [0, m) (the v1 vector sum up to a
+    // few above), but host arithmetic also leaves values a little below zero, and a caller may store
+    // any int of the class. A product takes a residue below 2^(mus + 1) as it is (mulmod_i) and a
+    // sum one below m (combine); a number with another residue is reduced first, behind a branch
+    // that costs the usual numbers an OR a residue and operand for products and a compare for sums.
+    template <int CNT>
+    __device__ __forceinline__ void reduce(int *x, int *y, int r0, const DevConsts *c) const {
+        if constexpr (L == 1 && !INL) {  // out of line: inlined in every step it doubled the steps' code
+            int t[CNT], u[CNT];          // memory of their own: the residues stay in registers
+#pragma unroll
+            for (int r = 0; r < CNT; r++) {
+                t[r] = x[r];
+                u[r] = y ? y[r] : 0;
+            }
+            ool_reduce(k.C, t, u, r0, CNT);
+#pragma unroll
+            for (int r = 0; r < CNT; r++) {
+                x[r] = t[r];
+                if (y) y[r] = u[r];
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < CNT; r++) {
+                x[r] = modd((double)x[r], md(r0 + r, c), mv(r0 + r, c));
+                if (y) y[r] = modd((double)y[r], md(r0 + r, c), mv(r0 + r, c));
+            }
+        }
+    }
+    __device__ __forceinline__ bool wide(uint32_t any) const { return (any >> (mus + 1)) != 0; }
+    // residues of x and y, fit for products (y may be null)
+    template <int CNT>
+    __device__ __forceinline__ void factors(int *x, int *y, int r0, const DevConsts *c) const {
+        uint32_t any = 0;
+#pragma unroll
+        for (int r = 0; r < CNT; r++) any |= (uint32_t)x[r] | (y ? (uint32_t)y[r] : 0u);
+        if (wide(any)) reduce<CNT>(x, y, r0, c);
+    }
+    // residues of x and y in [0, m)
+    __device__ __forceinline__ void canonical(int *x, int *y, const DevConsts *c) const {
+        bool out = false;
+#pragma unroll
+        for (int r = 0; r < R; r++)
+            out |= (unsigned)x[r] >= (unsigned)mi(r, c) || (unsigned)y[r] >= (unsigned)mi(r, c);
+        if (out) reduce<R>(x, y, 0, c);
+    }
+    // The element kernels that cold_round names only ask (COLD = false), and leave the reduction to the
+    // function that does a number again: FACTORS: x and y fit for a product; otherwise x in [0, m)
+    template <bool COLD>
+    static constexpr bool ASKS = cold_round(N, L) && !COLD;
+    template <bool FACTORS>
+    __device__ __forceinline__ bool unfit(const MP<R> &x, const MP<R> &y) const {
+        bool out = false;
+        if constexpr (FACTORS) {
+            uint32_t any = 0;
+#pragma unroll
+            for (int r = 0; r < R; r++) any |= (uint32_t)x.d[r] | (uint32_t)y.d[r];
+            out = wide(any);
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; r++) out |= (unsigned)x.d[r] >= (unsigned)mi(r);
+        }
+        return xlane_usum<L>(out ? 1u : 0u) != 0;
     }
     __device__ __forceinline__ int prow(int g) const { return g > k.C->log2m ? k.C->log2m : g; }
     __device__ __forceinline__ Er unit_low() const { return Er{k.C->unit_low.frac, k.C->unit_low.exp}; }
@@ -417,11 +490,17 @@ struct Grp {
         const Er xl{x.ev0.frac * (double)nzx, x.ev0.exp + gamma}, xu{x.ev1.frac * (double)nzx, x.ev1.exp + gamma};
         const Er yl{y.ev0.frac * (double)nzy, y.ev0.exp + theta}, yu{y.ev1.frac * (double)nzy, y.ev1.exp + theta};
         int lx[R], ly[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            lx[r] = x.d[r];
+            ly[r] = y.d[r];
+        }
+        factors<R>(lx, ly, 0, k.C);
         const int *rg = k.P2 + (size_t)prow(gamma) * N, *rt = k.P2 + (size_t)prow(theta) * N;
 #pragma unroll
         for (int r = 0; r < R; r++) {
-            lx[r] = nzx ? mmul(x.d[r], rg[ix(r)], r) : 0;
-            ly[r] = nzy ? mmul(y.d[r], rt[ix(r)], r) : 0;
+            lx[r] = nzx ? mmul(lx[r], rg[ix(r)], r) : 0;
+            ly[r] = nzy ? mmul(ly[r], rt[ix(r)], r) : 0;
         }
         const int c = rns_cmp_ev(lx, xl, xu, ly, yl, yu);
         if constexpr (ABS) {
@@ -436,8 +515,15 @@ struct Grp {
     // cuda::rns_cmp(x, y) on bare residues, src/rns.cuh:1242-1260: both evaluations computed
     __device__ __forceinline__ int rns_cmp(const int *dx, const int *dy) const {
         Er xl, xu, yl, yu;
-        eval_full(dx, xl, xu);
-        eval_full(dy, yl, yu);
+        int cx[R], cy[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            cx[r] = dx[r];
+            cy[r] = dy[r];
+        }
+        canonical(cx, cy, k.C);
+        eval_full(cx, xl, xu);
+        eval_full(cy, yl, yu);
         return rns_cmp_ev(dx, xl, xu, dy, yl, yu);
     }
 
@@ -479,14 +565,22 @@ struct Grp {
     }
 
     // cuda::mp_add (mp_add_common + rounding), src/arith/add.cuh:126-200
-    template <bool RND = true>
+    // CHECK = false: residues known to be in [0, m)
+    template <bool RND = true, bool CHECK = true>
     __device__ __forceinline__ void add(MP<R> &res, const MP<R> &x, const MP<R> &y) const {
         const Align a = align(x, y);
+        int xd[R], yd[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            xd[r] = x.d[r];
+            yd[r] = y.d[r];
+        }
+        if constexpr (CHECK) canonical(xd, yd, k.C);
         Er e0, e1;
         er_add_pair(a.sx ? a.x1 : a.x0, a.sy ? a.y1 : a.y0, a.sx ? a.x0 : a.x1, a.sy ? a.y0 : a.y1, e0, e1);
         int sign = e0.frac < 0;
         if (sign != (e1.frac < 0)) {
-            sign = sign_estimate(x.d, y.d, a.sx, a.sy, a.gamma, a.theta, a.nzx, a.nzy);
+            sign = sign_estimate(xd, yd, a.sx, a.sy, a.gamma, a.theta, a.nzx, a.nzy);
             const Er u{k.C->unit_low.frac * (double)(1 - 2 * sign), k.C->unit_low.exp};
             if (sign)
                 e1 = u;
@@ -498,7 +592,7 @@ struct Grp {
         const int row = prow(sh);
         const int fs = shx ? a.fx : a.fy, fo = shx ? a.fy : a.fx;
 #pragma unroll
-        for (int r = 0; r < R; r++) res.d[r] = combine(x.d[r], y.d[r], row, shx, sh != 0, fs, fo, sign, r, k.C);
+        for (int r = 0; r < R; r++) res.d[r] = combine(xd[r], yd[r], row, shx, sh != 0, fs, fo, sign, r, k.C);
         finish_add<RND>(res, a, e0, e1, sign);
     }
     template <bool RND>
@@ -526,11 +620,18 @@ struct Grp {
         res.ev1 = p.ev1;
     }
     // cuda::mp_mul, src/arith/mul.cuh:53-74
-    template <bool RND = true>
+    template <bool RND = true, bool CHECK = true>
     __device__ __forceinline__ void mul(MP<R> &res, const MP<R> &x, const MP<R> &y) const {
+        int xd[R], yd[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            xd[r] = x.d[r];
+            yd[r] = y.d[r];
+        }
+        if constexpr (CHECK) factors<R>(xd, yd, 0, k.C);
         mul_scalars(res, x.sign, x.exp, x.ev0, x.ev1, y.sign, y.exp, y.ev0, y.ev1);
 #pragma unroll
-        for (int r = 0; r < R; r++) res.d[r] = mmul(x.d[r], y.d[r], r);
+        for (int r = 0; r < R; r++) res.d[r] = mmul(xd[r], yd[r], r);
         if constexpr (RND) round_if_needed(res);
     }
 
@@ -546,11 +647,15 @@ struct Grp {
         return sig;
     }
     // cuda::mp_mul_d, src/arith/muld.cuh:59-73
-    template <bool RND = true>
+    template <bool RND = true, bool CHECK = true>
     __device__ __forceinline__ void mul_d(MP<R> &res, const MP<R> &x, double y) const {
+        int xd[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) xd[r] = x.d[r];
+        if constexpr (CHECK) factors<R>(xd, nullptr, 0, k.C);
         const double sig = muld_scalars(res, x.sign, x.exp, x.ev0, x.ev1, y);
 #pragma unroll
-        for (int r = 0; r < R; r++) res.d[r] = mmul(x.d[r], modd(sig, md(r), mv(r)), r);
+        for (int r = 0; r < R; r++) res.d[r] = mmul(xd[r], modd(sig, md(r), mv(r)), r);
         if constexpr (RND) round_if_needed(res);
     }
 
@@ -595,31 +700,45 @@ struct Grp {
         const double sig = muld_scalars(p, xs, xe, x0, x1, y);
         return step_tail<FULL>(acc, p, dx, nullptr, sig, true);
     }
-    // residue r of the product: x_r * y_r, or x_r * (sig mod m_r) for a double factor
-    __device__ __forceinline__ int prod_digit(const int *dx, const int *dy, double sig, bool dbl, int r,
-                                              const DevConsts *c) const {
-        return dbl ? mmul(dx[r], modd(sig, md(r, c), mv(r, c)), r, c) : mmul(dx[r], dy[r], r, c);
+    // the product's residues, x_r * y_r, or x_r * (sig mod m_r) for a double factor: f(r, residue).
+    // In runs of four, which bounds the operands held at once
+    template <class F>
+    __device__ __forceinline__ void product(const int *dx, const int *dy, double sig, bool dbl, const DevConsts *c,
+                                            F &&f) const {
+        constexpr int RUN = R < 4 ? R : 4;
+#pragma unroll
+        for (int r0 = 0; r0 < R; r0 += RUN) {
+            int x[RUN], y[RUN];
+#pragma unroll
+            for (int r = 0; r < RUN; r++) {
+                x[r] = dx[r0 + r];
+                y[r] = dbl ? 0 : dy[r0 + r];
+            }
+            factors<RUN>(x, dbl ? nullptr : y, r0, c);
+#pragma unroll
+            for (int r = 0; r < RUN; r++)
+                f(r0 + r, mmul(x[r], dbl ? modd(sig, md(r0 + r, c), mv(r0 + r, c)) : y[r], r0 + r, c));
+        }
     }
     template <bool FULL>
     __device__ __forceinline__ bool step_tail(MP<R> &acc, MP<R> &p, const int *dx, const int *dy, double sig,
                                               bool dbl) const {
-        if (needs_round(p)) {
-            if constexpr (!FULL) return false;
-#pragma unroll
-            for (int r = 0; r < R; r++) p.d[r] = prod_digit(dx, dy, sig, dbl, r, k.C);
-            round_if_needed(p);
-            add(acc, acc, p);
-            return true;
+        // the product needs rounding, or the sum's interval straddles zero
+        bool slow = needs_round(p);
+        Align a{};
+        Er e0{}, e1{};
+        int sign = 0;
+        if (!slow) {
+            a = align(acc, p);
+            er_add_pair(a.sx ? a.x1 : a.x0, a.sy ? a.y1 : a.y0, a.sx ? a.x0 : a.x1, a.sy ? a.y0 : a.y1, e0, e1);
+            sign = e0.frac < 0;
+            slow = sign != (e1.frac < 0);
         }
-        const Align a = align(acc, p);
-        Er e0, e1;
-        er_add_pair(a.sx ? a.x1 : a.x0, a.sy ? a.y1 : a.y0, a.sx ? a.x0 : a.x1, a.sy ? a.y0 : a.y1, e0, e1);
-        const int sign = e0.frac < 0;
-        if (sign != (e1.frac < 0)) {
+        if (slow) {
             if constexpr (!FULL) return false;
-#pragma unroll
-            for (int r = 0; r < R; r++) p.d[r] = prod_digit(dx, dy, sig, dbl, r, k.C);
-            add(acc, acc, p);
+            product(dx, dy, sig, dbl, k.C, [&](int r, int v) { p.d[r] = v; });
+            round_if_needed(p);
+            add<true, false>(acc, acc, p);
             return true;
         }
         const bool shx = a.gamma > 0;
@@ -627,9 +746,8 @@ struct Grp {
         const int row = prow(sh);
         const int fs = shx ? a.fx : a.fy, fo = shx ? a.fy : a.fx;
         const DevConsts *c = fresh<!FULL>();
-#pragma unroll
-        for (int r = 0; r < R; r++)
-            acc.d[r] = combine(acc.d[r], prod_digit(dx, dy, sig, dbl, r, c), row, shx, sh != 0, fs, fo, sign, r, c);
+        product(dx, dy, sig, dbl, c,
+                [&](int r, int v) { acc.d[r] = combine(acc.d[r], v, row, shx, sh != 0, fs, fo, sign, r, c); });
         acc.sign = sign;
         acc.exp = (a.ex == 0) ? a.ey : a.ex;
         if (sign) {
@@ -645,11 +763,11 @@ struct Grp {
         }
         return true;
     }
-    // generic addition that may refuse the rare paths (see fma_step)
+    // addition of sums that may refuse the rare paths (see fma_step)
     template <bool FULL>
     __device__ __forceinline__ bool add_try(MP<R> &res, const MP<R> &x, const MP<R> &y) const {
         if constexpr (FULL) {
-            add(res, x, y);
+            add<true, false>(res, x, y);
             return true;
         } else {
             const Align a = align(x, y);

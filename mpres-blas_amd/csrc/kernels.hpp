@@ -299,16 +299,21 @@ __global__ __launch_bounds__(BLK) void k_sqrt(const DevConsts *__restrict__ C, i
 template <int N, int L, int OP, bool COLD>
 __device__ __forceinline__ bool elem_one(const DevConsts *__restrict__ C, AoSRef<N> x, AoSRef<N> y,
                                          const double *__restrict__ yd, AoSRef<N> r, long long i) {
-    Grp<N, L> g(C);
+    using G = Grp<N, L>;
+    constexpr bool ASKS = G::template ASKS<COLD>;
+    G g(C);
     MP<N / L> a, b, c;
     load_aos(g, a, x, i);
     if (OP == 3) {
-        g.template mul_d<false>(c, a, yd[i]);
+        if (ASKS && g.template unfit<true>(a, a)) return g.lane() == 0;
+        g.template mul_d<false, !ASKS>(c, a, yd[i]);
     } else {
         load_aos(g, b, y, i);
+        if (ASKS && OP < 2 && (g.template unfit<false>(a, a) || g.template unfit<false>(b, b))) return g.lane() == 0;
+        if (ASKS && OP == 2 && g.template unfit<true>(a, b)) return g.lane() == 0;
         if (OP == 1) b.sign ^= 1;  // mp_sub, src/arith/sub.cuh:41-53
-        if (OP < 2) g.template add<false>(c, a, b);
-        if (OP == 2) g.template mul<false>(c, a, b);
+        if (OP < 2) g.template add<false, !ASKS>(c, a, b);
+        if (OP == 2) g.template mul<false, !ASKS>(c, a, b);
         if (OP == 4) g.template vadd<false>(c, a, b);
     }
     if (g.template round_fails<COLD>(c)) return g.lane() == 0;
@@ -452,7 +457,7 @@ __global__ __launch_bounds__(BLK) void k_tree(const DevConsts *__restrict__ C, A
                 MP<N / L> a, c, r;
                 load_aos(g, a, part, base + t);
                 load_aos(g, c, part, base + t + s);
-                g.add(r, a, c);
+                g.template add<true, false>(r, a, c);  // partial sums of this library
                 store_aos(g, r, part, base + t);
             }
         }
@@ -503,8 +508,10 @@ __device__ __forceinline__ bool axpy_one(const DevConsts *__restrict__ C, const 
     load_soa(g, a, alpha, 0);
     load_soa(g, xv, x, ix);
     load_soa(g, yv, y, iy);
-    g.template mul<false>(r, xv, a);
-    bool full = g.template round_fails<COLD>(r);
+    constexpr bool ASKS = Grp<N, L>::template ASKS<COLD>;
+    bool full = ASKS && g.template unfit<true>(xv, a);
+    g.template mul<false, !ASKS>(r, xv, a);
+    full |= g.template round_fails<COLD>(r);
     g.template vadd<false>(r, r, yv);
     full |= g.template round_fails<COLD>(r);
     if (full) return g.lane() == 0;
@@ -537,9 +544,11 @@ __device__ __forceinline__ bool axpy_v2_one(const DevConsts *__restrict__ C, AoS
     if (NEG) a.sign ^= 1;
     load_aos(g, xv, x, i);
     load_aos(g, yv, y, i);
-    g.template mul<false>(s, a, xv);
-    bool full = g.template round_fails<COLD>(s);
-    g.template add<false>(s, s, yv);
+    constexpr bool ASKS = Grp<N, L>::template ASKS<COLD>;
+    bool full = ASKS && (g.template unfit<true>(a, xv) || g.template unfit<false>(yv, yv));
+    g.template mul<false, !ASKS>(s, a, xv);
+    full |= g.template round_fails<COLD>(s);
+    g.template add<false, !ASKS>(s, s, yv);
     full |= g.template round_fails<COLD>(s);
     if (full) return g.lane() == 0;
     store_aos(g, s, r, i);
@@ -696,7 +705,7 @@ __global__ __launch_bounds__(BLK) ELEM_WAVES(N, L) void k_gemm_fin(const DevCons
     g.template mul<false>(r, cv, b);
     g.round_here(r);
     if constexpr (V2)
-        g.template add<false>(r, s2, r);
+        g.template add<false, false>(r, s2, r);
     else
         g.template vadd<false>(r, r, s2);
     g.round_here(r);

@@ -48,7 +48,7 @@ __device__ void batch_tree(const Grp<N, L> &g, AoSRef<N> part, long long nb, int
                 MP<N / L> a, c, r;
                 load_aos(g, a, part, blk * b + t);
                 load_aos(g, c, part, blk * b + t + s);
-                g.add(r, a, c);
+                g.template add<true, false>(r, a, c);  // partial sums of this kernel
                 store_aos(g, r, part, blk * b + t);
             }
         }

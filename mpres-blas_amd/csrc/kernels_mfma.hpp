@@ -141,6 +141,7 @@ k_mf_prescale(const DevConsts *__restrict__ C, int cnt, int JP, int k, int KP, i
         const int *dig = digits_of<N>(X, idx);
         for (int r = 0; r < N; r++) x[r] = dig[r];
     }
+    for (int r = 0; r < N; r++) x[r] = pos_reduce(x[r], C->m[r]);
     if (up.frac == 0 || -d > C->log2m + 1) {
         // zero, or truncated to zero (X < M < 2^(log2m + 1))
         for (int r = 0; r < N; r++) x[r] = 0;

@@ -378,10 +378,10 @@ MPH_HD int mulmod_c(uint32_t a, uint32_t w, uint32_t wq, uint32_t m) {
     const uint32_t r = a * w - q * m, s = r - m;
     return (int)(r < s ? r : s);
 }
-// (a * b) mod m for 0 <= a, b < m, 2^s <= m < 1.43e9 (so 3 m < 2^32, s <= 30), mu = floor(2^(s + 32) / m):
-// q = floor(floor(a b / 2^s) mu / 2^32) is the quotient, or up to two less (the first floor costs
-// less than 2^s / m <= 1, mu's less than a b / 2^(s + 32) <= 1), so a b - q m (mod 2^32) lies in
-// [0, 3m). Nine integer instructions, all full rate, where mulmod takes about eighteen.
+// (a * b) mod m for a, b < 2^(s + 1), 2^s <= m < 2^(s + 1), m < 1.43e9 (so 3 m < 2^32, s <= 30), mu =
+// floor(2^(s + 32) / m): q = floor(floor(a b / 2^s) mu / 2^32) is the quotient, or up to two less (the
+// first floor costs less than 2^s / m <= 1, mu's less than a b / 2^(s + 32) <= 1), so a b - q m (mod
+// 2^32) lies in [0, 3m). Nine integer instructions, all full rate, where mulmod takes about eighteen.
 MPH_HD int mulmod_i(uint32_t a, uint32_t b, uint32_t m, uint32_t mu, int s) {
     const uint64_t p = (uint64_t)a * b;
 #if defined(__HIP_DEVICE_COMPILE__)

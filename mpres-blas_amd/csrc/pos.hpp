@@ -18,7 +18,7 @@
 // the original operands' evaluations. Results equal the residue chain's bit for bit.
 //
 // Operands must be normalised as every operation leaves them: X / M below 2^(mp_h + 1) and
-// the evaluation within a relative 2^-20 of X / M. Chains with others (PosOp::bad) and chains
+// the evaluation within a relative 2^-20 of X / M, residues not below zero. Chains with others (PosOp::bad) and chains
 // that cancel exactly to zero are left to the residue kernels.
 #pragma once
 
@@ -120,6 +120,9 @@ template <int N>
 __device__ __forceinline__ void pos_operand(const DevConsts *__restrict__ C, const int *d, int s, int e, Er e0, Er e1,
                                             PosOp<Pos<N>::W> &o) {
     constexpr int W = Pos<N>::W;
+    uint32_t any = 0;  // its top bit: a residue below zero, which pos_from_digits does not take
+#pragma unroll
+    for (int r = 0; r < N; r++) any |= (uint32_t)d[r];
     pos_from_digits<N, W, true>(C, d, o.x);
     o.e = e;
     o.s = s;
@@ -129,7 +132,7 @@ __device__ __forceinline__ void pos_operand(const DevConsts *__restrict__ C, con
     const bool zero = o.h == 0;
     const bool fits = e1.exp <= pos_const(C->mp_h) && u >= f * (1 - 0x1p-44) && u <= f * (1 + POS_GIVEN) &&
                       l <= f * (1 + 0x1p-44) && l >= f * (1 - POS_GIVEN);
-    o.bad = zero ? (e1.frac != 0 || e0.frac != 0) : !fits;
+    o.bad = (int)any < 0 || (zero ? (e1.frac != 0 || e0.frac != 0) : !fits);
 }
 template <int W>
 __device__ __forceinline__ PosOp<W> pos_unpack(const PosRec<W> &r) {

@@ -80,7 +80,7 @@ __device__ __forceinline__ int pos_reduce(int d, int m) {
     const int v = d % m;
     return v < 0 ? v + m : v;
 }
-// The integer of residues: X = sum c_i M/m_i - rank M with c_i = |x_i w_i| mod m_i, its low WX
+// The integer of residues (any int from 0 of the class): X = sum c_i M/m_i - rank M with c_i = |x_i w_i| mod m_i, its low WX
 // words. NORM: X / M below 2^-40, and rank the nearest integer of sum c_i / m_i; otherwise any
 // X < M (WX = N: all of it): rank is the whole part of a sum that may be off by 2^-40, so the
 // result is brought into [0, M). Columns of 28-bit limbs in 64 bits: N products below 2^59 and a carry

@@ -698,7 +698,8 @@ static int dot_common(mpres_ctx_t *c, WsUse &wu, int mode, int n, SoA xs, int in
         else
             HIPCHK(o->fold(c->dev, mode, 0, n, G, xs, incx, ys, incy, xa, ya, p1, st));
     }
-    if (pos || c->host.n > 8) HIPCHK(o->fold(c->dev, mode, 1, n, G, xs, incx, ys, incy, xa, ya, p1, st));
+    if (pos ? c->pos->leaves(G) : c->host.n > 8)
+        HIPCHK(o->fold(c->dev, mode, 1, n, G, xs, incx, ys, incy, xa, ya, p1, st));
     HIPCHK(o->tree(c->dev, p1, b3, P, g3, p2, st));
     // pass 2: one block of b3 over the g3 block results (src/mpreduct.cuh:81-112)
     SoA none{};
@@ -994,10 +995,11 @@ int mpres_gemv(mpres_ctx_t *c, int trans, int m, int n, const mp_array_t *alpha,
     HIPCHK(o->gemv_fold(c->dev, tr, 3, m, n, soa_of(A), lda, bx, b3, nvt, part, aux, strm(st)));
     if (c->pos) {
         if (rec) HIPCHK(c->pos->records(c->dev, 0, 0, lx, 1, SoA{}, bx, false, lx, rec, strm(st)));
-        ProfScope ps(c, c->host.n > 8 ? -1 : (int)OP_GEMV, strm(st));
+        ProfScope ps(c, OP_GEMV, strm(st));
         HIPCHK(c->pos->gemv(c->dev, tr, m, n, soa_of(A), lda, bx, rec, b3, nvt, part, strm(st)));
     }
-    HIPCHK(o->gemv_fold(c->dev, tr, 4, m, n, soa_of(A), lda, bx, b3, nvt, part, aux, strm(st)));
+    if (!c->pos || c->pos->leaves(nvt))
+        HIPCHK(o->gemv_fold(c->dev, tr, 4, m, n, soa_of(A), lda, bx, b3, nvt, part, aux, strm(st)));
     HIPCHK(o->tree(c->dev, part, b3, next_pow2((unsigned)b3), ly, sums, strm(st)));
     HIPCHK(o->gemv_final(c->dev, ly, ys, incy, sums, strm(st)));
     return MPRES_OK;
@@ -1055,7 +1057,7 @@ int mpres_gemm(mpres_ctx_t *c, int ta, int tb, int m, int n, int k, const mp_arr
             ProfScope ps(c, OP_GEMM, strm(st));
             HIPCHK(c->pos->gemm(c->dev, 0, 0, m, n, k, soa_of(A), lda, soa_of(B), ldb, ra, rb, w, strm(st)));
         }
-        for (int pass = 3; pass < 5; pass++)
+        for (int pass = c->pos->gemm_leaves((long long)m * n) ? 3 : 4; pass < 5; pass++)
             HIPCHK(o->gemm(c->dev, pass, c->bits, m, n, k, soa_of(alpha), soa_of(A), lda, soa_of(B), ldb, soa_of(beta),
                            soa_of(C), ldc, w, ra, strm(st)));
         return MPRES_OK;
@@ -1132,6 +1134,7 @@ int mpres_gemm_v2(mpres_ctx_t *c, int ta, int tb, int m, int n, int k, const voi
         if (pass == 3 && c->pos)
             HIPCHK(c->pos->gemm_v2(c->dev, tra, trb, m, n, k, (const char *)A, lda, (const char *)B, ldb, ra, rb, w,
                                    strm(st)));
+        if (pass == 3 && c->pos && !c->pos->gemm_leaves((long long)m * n)) continue;
         HIPCHK((pass == 4 ? epilogue_ops(c, o, (long long)m * n) : o)->gemm_v2(c->dev, pass, c->bits, tra, trb, m, n, k, (const char *)alpha, (const char *)A,
                                         lda, (const char *)B, ldb, (const char *)beta, (char *)C, ldc, w, ra,
                                         pass == 0 ? fk.s1 : strm(st)));

@@ -67,7 +67,7 @@ struct Ops {
                       hipStream_t);
     // the reduction launchers take a pass: 0 = main kernel (over 8 moduli only the short chains of dot: the
     // others are PosOps'), 1 = fixup kernel (see kernels.hpp);
-    // gemv_fold runs passes 0..3 and gemm / gemm_v2 passes 0..4 (see launch.hpp)
+    // gemv_fold runs passes 0..4 and gemm / gemm_v2 passes 0..4 (see launch.hpp)
     hipError_t (*fold)(const DevConsts *, int, int, long long, long long, SoA, int, SoA, int, const char *,
                        const char *, char *, hipStream_t);
     hipError_t (*tree)(const DevConsts *, char *, int, unsigned, int, char *, hipStream_t);
@@ -113,9 +113,11 @@ struct Ops {
     hipError_t (*batch)(const DevConsts *, const BatchItem *, int, int *, char *, int, hipStream_t);
 };
 
-// The reduction chains on positional integers (kernels_pos.hpp), over 8 moduli. What they cannot do
-// they mark REDO for the residue kernels' fixup pass.
+// The reduction chains on positional integers (kernels_pos.hpp), over 8 moduli.
 struct PosOps {
+    // whether that many chains (fold and gemv; gemm) may leave some, marked REDO, to the residue kernels'
+    // fixup pass
+    bool (*leaves)(long long), (*gemm_leaves)(long long);
     hipError_t (*fold)(const DevConsts *, int, long long, long long, SoA, int, SoA, int, const char *, const char *,
                        char *, hipStream_t);
     size_t (*rec_bytes)(long long);

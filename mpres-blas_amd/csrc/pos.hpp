@@ -19,7 +19,7 @@
 //
 // Operands must be normalised as every operation leaves them: X / M below 2^(mp_h + 1) and
 // the evaluation within a relative 2^-20 of X / M, residues not below zero. Chains with others (PosOp::bad) and chains
-// that cancel exactly to zero are left to the residue kernels.
+// that cancel exactly to zero are left to the residue arithmetic (kernels_pos.hpp).
 #pragma once
 
 #include "bigint.hpp"
@@ -413,7 +413,7 @@ __device__ __forceinline__ void pos_snap_zero(PosSnap<W> &s) {
     s.lazy = false;
 }
 // The evaluation after `to` terms. The terms since the snapshot were added without rounding and
-// without a straddling interval, so the scalar fields alone are replayed.
+// without a straddling interval, so the scalar fields alone are replayed, each term's loaded a step ahead.
 template <int N, bool U, class PV>
 __device__ __forceinline__ void pos_replay(const DevConsts *__restrict__ C, const PV &pv, PosSnap<Pos<N>::W> &s,
                                         long long to) {
@@ -421,9 +421,13 @@ __device__ __forceinline__ void pos_replay(const DevConsts *__restrict__ C, cons
         pos_eval<N, U>(C, s.x, s.v.ev0, s.v.ev1);
         s.lazy = false;
     }
+    if (s.at >= to) return;
+    typename PV::Scalars cur = pv.scalars(s.at);
     for (; s.at < to; s.at++) {
+        const typename PV::Scalars nxt = pv.scalars(s.at + 1 < to ? s.at + 1 : s.at);
         Sc p;
-        pv.template scalars<U>(C, s.at, p);
+        pv.template product<U>(C, s.at, cur, p);
+        cur = nxt;
         const Align a = align_sc(pos_const(C->mp_j), s.v.sign, s.v.exp, s.v.ev0, s.v.ev1, p.sign, p.exp, p.ev0, p.ev1);
         Er e0, e1;
         er_add_pair(a.sx ? a.x1 : a.x0, a.sy ? a.y1 : a.y0, a.sx ? a.x0 : a.x1, a.sy ? a.y0 : a.y1, e0, e1);
@@ -457,6 +461,8 @@ __device__ __noinline__ bool pos_step_exact(const DevConsts *__restrict__ C, con
     pv.template exact<false>(C, at, p);
     pos_add_exact<N, false>(C, v, p);
     pos_from_exact<N>(C, v, acc);
+#pragma unroll
+    for (int i = 0; i < W; i++) snap.x[i] = acc.x[i];
     snap.v = Sc{v.s, v.e, v.ev0, v.ev1};
     snap.at = at + 1;
     snap.lazy = false;
@@ -560,6 +566,10 @@ struct PosTerms {
         else
             pos_operand<N>(C, o.d, o.s, o.e, o.e0, o.e1, x);
     }
+    // the same terms, the operands as they lie in memory
+    __device__ __forceinline__ PosTerms<N, VX, VY, false, false> plain() const {
+        return {X, Y, nullptr, nullptr, x0, dx, y0, dy, 0, 0, 0, 0};
+    }
     __device__ __forceinline__ Raw load(long long k) const {
         Raw o;
         load1(X, x0 + k * dx, rx, rx0 + k * rdx, o.x);
@@ -584,15 +594,22 @@ struct PosTerms {
         scalars_of<N>(Y, y0 + k * dy, s, e, b0, b1);
         pos_mul_exact<N, U>(C, x, a0, a1, y, b0, b1, p);
     }
-    // sign, exponent and evaluation of term k
-    template <bool U>
-    __device__ __forceinline__ void scalars(const DevConsts *__restrict__ C, long long k, Sc &p) const {
+    struct Scalars {
         int xs, xe, ys, ye;
         Er a0, a1, b0, b1;
-        scalars_of<N>(X, x0 + k * dx, xs, xe, a0, a1);
-        scalars_of<N>(Y, y0 + k * dy, ys, ye, b0, b1);
+    };
+    __device__ __forceinline__ Scalars scalars(long long k) const {
+        Scalars o;
+        scalars_of<N>(X, x0 + k * dx, o.xs, o.xe, o.a0, o.a1);
+        scalars_of<N>(Y, y0 + k * dy, o.ys, o.ye, o.b0, o.b1);
+        return o;
+    }
+    // sign, exponent and evaluation of term k from its operands' fields
+    template <bool U>
+    __device__ __forceinline__ void product(const DevConsts *__restrict__ C, long long k, const Scalars &o,
+                                            Sc &p) const {
         const ScC K = sc_consts(C);
-        sc_mul(K, p, xs, xe, a0, a1, ys, ye, b0, b1);
+        sc_mul(K, p, o.xs, o.xe, o.a0, o.a1, o.ys, o.ye, o.b0, o.b1);
         if (sc_needs_round(K, p.ev1)) {
             PosExact<W> q;
             exact<U>(C, k, q);

@@ -4,6 +4,7 @@ import ctypes as C
 import importlib.util
 import os
 
+import numpy as np
 import pytest
 
 import pyoracle as po
@@ -56,4 +57,21 @@ def test_quiet_reductions(name, kind):
                           C.byref(db), C.byref(dC), m, None, 0, None))
     want = o.gemm(m, n, k, al, A, m, B, k, be, Cm, m, D)
     assert c.array_to_host(dC, m * n).tobytes() == want.tobytes()
+    c.close()
+
+
+@pytest.mark.parametrize("name", ["16_4double", "32_8double"])
+def test_sparse_gemm(name):
+    """split-form gemm on sparse operands with zeros of both signs: entries whose every product is zero"""
+    c, o, r = mp.Context(name), po.Oracle(name), np.random.default_rng(5)
+    for m, n, k in ((64, 20, 17), (70, 65, 33)):
+        print(f"[case] sparse gemm {name} {m}x{n}x{k}", flush=True)
+        A, B, Cm = (o.set_d(np.where(r.uniform(0, 1, q) < 0.1, r.standard_normal(q), r.choice([0.0, -0.0], q)), D)
+                    for q in (m * k, k * n, m * n))
+        al, be = o.set_d([1.5], D), o.set_d([-1.0], D)
+        dA, dB, dC, da, db = (c.array_from_host(v) for v in (A, B, Cm, al, be))
+        mp.check(c.L.mpres_gemm(c.h, mp.NO_TRANS, mp.NO_TRANS, m, n, k, C.byref(da), C.byref(dA), m, C.byref(dB), k,
+                                C.byref(db), C.byref(dC), m, None, 0, None))
+        want = o.gemm(m, n, k, al, A, m, B, k, be, Cm, m, D)
+        assert c.array_to_host(dC, m * n).tobytes() == want.tobytes()
     c.close()

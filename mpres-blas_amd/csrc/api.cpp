@@ -1331,12 +1331,25 @@ int mpres_batch_plan(mpres_ctx_t *c, const mpres_batch_problem_t *probs, int cou
     if (rc) return fail(rc, "%s", lay.err.c_str());
     if (ws && wsb < lay.ws_bytes)
         return fail(MPRES_ERR_WORKSPACE, "workspace of %zu bytes, %zu needed", wsb, lay.ws_bytes);
+    char *own = nullptr;
+    if (!ws && lay.ws_bytes) {
+        hipError_t e = hipMalloc(&own, lay.ws_bytes);
+        if (e != hipSuccess && groups) {  // likewise with the memory that there is
+            (void)hipGetLastError();
+            rc = batch_layout(probs, count, c->host.n, u.gemv_rows, lay);
+            if (rc) return fail(rc, "%s", lay.err.c_str());
+            e = hipMalloc(&own, lay.ws_bytes);
+        }
+        if (e != hipSuccess) return fail(MPRES_ERR_HIP, "hipMalloc(batch scratch): %s", hipGetErrorString(e));
+    }
     auto *b = new mpres_batch();
     b->ctx = c;
     b->ops = o;
     b->count = (int)lay.items.size();
     b->fmas = lay.fmas;
     b->used = u;
+    b->ws = own ? own : (char *)ws;
+    b->own_ws = own != nullptr;
     *plan = b;
     if (b->count == 0) return MPRES_OK;
     auto bail = [&](const char *what, hipError_t e) {
@@ -1345,12 +1358,6 @@ int mpres_batch_plan(mpres_ctx_t *c, const mpres_batch_problem_t *probs, int cou
         return fail(MPRES_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
     };
     hipError_t e;
-    if (ws) {
-        b->ws = (char *)ws;
-    } else if (lay.ws_bytes) {
-        if ((e = hipMalloc(&b->ws, lay.ws_bytes)) != hipSuccess) return bail("hipMalloc(batch scratch)", e);
-        b->own_ws = true;
-    }
     const size_t tbl = lay.items.size() * sizeof(BatchItem);
     const size_t qoff = (tbl + 255) / 256 * 256;
     if ((e = hipMalloc(&b->dmem, qoff + 256)) != hipSuccess) return bail("hipMalloc(batch items)", e);

@@ -40,15 +40,18 @@ constexpr size_t BATCH_WS_ALIGN = 256;
 // group of lanes of its workgroup (groups) a chain; the rows are split evenly. Every item forms
 // alpha * x again, which costs it lx products beside rows * lx. One gemv of 1024^2 over 16 moduli,
 // before in items of 128 rows: 17.2 -> 2.2 ms; 512 gemvs of 48 rows keep one item each (0.26 ms;
-// two each 0.34).
+// two each 0.34). Every item also holds its own copy of alpha * x: where a batch's copies, beyond those of
+// items of cap rows, would take more than BATCH_SPARE (wide gemvs: 512 x 32768 at 106 bits, an
+// item a row, 1.2 GB, as much as A), the parts are halved until they do not (parts).
 constexpr int BATCH_PARTS = 512;
-inline int batch_rows(double fmas, int lx, int ly, int block3, int groups, int cap) {
-    const double fair = std::ceil(fmas / BATCH_PARTS / lx);
-    const int least = std::max(1, (groups + block3 - 1) / block3);
+constexpr double BATCH_SPARE = 256.0 * (1 << 20);
+inline int batch_rows(double fmas, int parts_of, int lx, int ly, int block3, int groups, int cap) {
+    const double fair = std::ceil(fmas / parts_of / lx);
+    const int least = 1 + (groups - 1) / block3;
     int rows = fair < cap ? std::max((int)fair, least) : cap;
     rows = std::min(rows, cap);
-    const int parts = (ly + rows - 1) / rows;
-    return (ly + parts - 1) / parts;
+    const int parts = 1 + (ly - 1) / rows;
+    return 1 + (ly - 1) / parts;
 }
 // multiply-accumulates of a batch; costliest: index of the problem with the most (-1: none)
 inline double batch_fmas(const mpres_batch_problem_t *probs, int count, int &costliest) {
@@ -96,6 +99,19 @@ inline int batch_layout(const mpres_batch_problem_t *probs, int count, int n_mod
     std::vector<Work> v;
     int costliest;
     const double total = batch_fmas(probs, count, costliest);
+    int parts = BATCH_PARTS;
+    for (; groups > 0 && parts > 1; parts /= 2) {
+        double spare = 0;
+        for (int i = 0; i < count; i++) {
+            const mpres_batch_problem_t &p = probs[i];
+            if (p.op != MPRES_BATCH_GEMV || p.m <= 0 || p.n <= 0 || p.block3 <= 0) continue;
+            const bool tr = p.trans != MPRES_NO_TRANS;
+            const int lx = tr ? p.m : p.n, ly = tr ? p.n : p.m;
+            const auto items = [&](int rows) { return (double)(1 + (ly - 1) / rows); };
+            spare += (items(batch_rows(total, parts, lx, ly, p.block3, groups, gemv_rows)) - items(gemv_rows)) * lx;
+        }
+        if (spare * S <= BATCH_SPARE) break;
+    }
     for (int i = 0; i < count; i++) {
         const mpres_batch_problem_t &p = probs[i];
         if (p.op == MPRES_BATCH_DOT) {
@@ -130,7 +146,7 @@ inline int batch_layout(const mpres_batch_problem_t *probs, int count, int n_mod
             const bool tr = p.trans != MPRES_NO_TRANS;
             const int lx = tr ? p.m : p.n, ly = tr ? p.n : p.m;
             out.fmas += (double)p.m * p.n;
-            const int rows = groups > 0 ? batch_rows(total, lx, ly, p.block3, groups, gemv_rows) : gemv_rows;
+            const int rows = groups > 0 ? batch_rows(total, parts, lx, ly, p.block3, groups, gemv_rows) : gemv_rows;
             for (int r0 = 0; r0 < ly; r0 += rows) {
                 const int r1 = ly - r0 > rows ? r0 + rows : ly, h = r1 - r0;
                 Work w{};

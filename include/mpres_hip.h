@@ -444,8 +444,8 @@ typedef struct {
     mp_array_t *r;        /* dot: result (one number); gemv: unused */
 } mpres_batch_problem_t;
 /* Geometry of the persistent kernel. It never changes results; 0 = built-in choice: the
- * gemv lanes of the context, or one lane at 16 moduli where a gemv with many chains is the
- * costliest problem; 4 workgroups per CU; up to 128 rows, fewer in a batch whose work would
+ * gemv lanes of the context, or one lane at 16 moduli where gemvs with many chains are nearly all
+ * of the work; 4 workgroups per CU; up to 128 rows, fewer in a batch whose work would
  * not spread over the compute units in items of that size. */
 typedef struct {
     int lanes;            /* lanes per number (a value mpres_lanes_supported accepts) */

@@ -1260,19 +1260,9 @@ struct mpres_batch {
 
 namespace {
 
-// Lanes of a batch, where the caller leaves them to the plan. Over 16 moduli, one lane a number
-// (its roundings positional) if the costliest problem is a gemv with more chains than a workgroup has
-// lanes, the gemv lanes (4) otherwise: 1024 dots and gemvs of 32 to 1024 rows in 12.0 ms with
-// one lane and 23.7 with 4 (half as far spread operands, which round seldom: 6.5 and 7.7 ms); 512
-// dots of 16 x 64 chains 0.42 and 0.36 ms.
+// lanes of a batch, where the caller leaves them to the plan
 int batch_lanes(const mpres_ctx *c, const mpres_batch_problem_t *probs, int count) {
-    const int L = c->ops[OP_GEMV]->L;
-    int i;
-    if (c->host.n != 16 || !c->lt[OP_GEMV].builtin || batch_fmas(probs, count, i) <= 0) return L;
-    const mpres_batch_problem_t &p = probs[i];
-    if (p.op != MPRES_BATCH_GEMV) return L;
-    const int ly = p.trans == MPRES_NO_TRANS ? p.m : p.n;
-    return (double)ly * p.block3 > 256 ? 1 : L;
+    return c->host.n == 16 && c->lt[OP_GEMV].builtin && batch_one_lane(probs, count) ? 1 : c->ops[OP_GEMV]->L;
 }
 
 // groups: for batch_layout, 0 where the caller gave the rows per item

@@ -53,21 +53,29 @@ inline int batch_rows(double fmas, int parts_of, int lx, int ly, int block3, int
     const int parts = 1 + (ly - 1) / rows;
     return 1 + (ly - 1) / parts;
 }
-// multiply-accumulates of a batch; costliest: index of the problem with the most (-1: none)
-inline double batch_fmas(const mpres_batch_problem_t *probs, int count, int &costliest) {
-    double sum = 0, most = 0;
-    costliest = -1;
+// multiply-accumulates of a batch; wide: those of its gemvs with more chains than a workgroup has lanes
+inline double batch_fmas(const mpres_batch_problem_t *probs, int count, double &wide) {
+    double sum = 0;
+    wide = 0;
     for (int i = 0; probs && i < count; i++) {
         const mpres_batch_problem_t &p = probs[i];
-        const double f = p.op == MPRES_BATCH_DOT ? (p.n > 0 ? p.n : 0)
-                                                 : (p.m > 0 && p.n > 0 ? (double)p.m * p.n : 0);
+        const bool dot = p.op == MPRES_BATCH_DOT;
+        const double f = dot ? (p.n > 0 ? p.n : 0) : (p.m > 0 && p.n > 0 ? (double)p.m * p.n : 0);
         sum += f;
-        if (f > most) {
-            most = f;
-            costliest = i;
-        }
+        if (!dot && (double)(p.trans == MPRES_NO_TRANS ? p.m : p.n) * p.block3 > 256) wide += f;
     }
     return sum;
+}
+// Whether a batch over 16 moduli runs one lane a number, its roundings positional: where such gemvs are
+// nearly all of it (over 7/8). 1024 dots and gemvs of 32 to 1024 rows 11.9 ms with one lane, 23.7 with 4; 64
+// gemvs of 200 rows 0.52 and 0.83 ms (operands that seldom round 0.22 and 0.28). A dot of few chains leaves most
+// lanes of its workgroup idle and runs longer for one lane a number: 512 dots of 1 x 64 chains and one gemv of
+// 200 rows 0.64 and 0.27 ms, 1024 of them and 512 gemvs of 100 rows (0.77 of the work) 0.96 and 0.57 (rounding
+// 1.28 and 1.40).
+inline bool batch_one_lane(const mpres_batch_problem_t *probs, int count) {
+    double wide;
+    const double sum = batch_fmas(probs, count, wide);
+    return sum > 0 && wide > 0.875 * sum;
 }
 
 // Returns MPRES_OK, or MPRES_ERR_ARG with layout.err naming the first bad problem.
@@ -97,8 +105,8 @@ inline int batch_layout(const mpres_batch_problem_t *probs, int count, int n_mod
         size_t bytes;
     };
     std::vector<Work> v;
-    int costliest;
-    const double total = batch_fmas(probs, count, costliest);
+    double wide;
+    const double total = batch_fmas(probs, count, wide);
     int parts = BATCH_PARTS;
     for (; groups > 0 && parts > 1; parts /= 2) {
         double spare = 0;

@@ -461,7 +461,9 @@ size_t mpres_batch_workspace(const mpres_ctx_t *ctx, const mpres_batch_problem_t
 int mpres_batch_plan(mpres_ctx_t *ctx, const mpres_batch_problem_t *probs, int count,
                      const mpres_batch_tuning_t *tuning, void *ws, size_t ws_bytes, mpres_batch_t **plan);
 int mpres_batch_run(mpres_batch_t *plan, void *stream);
-/* multiply-accumulates of the batch (dot: n, gemv: m * n, summed) and the plan's item count */
+/* multiply-accumulates of the batch (dot: n, gemv: m * n, summed), the plan's item count, and its
+ * geometry: a plan of the same problems with that tuning is the same plan (gemv_rows 0: chosen for
+ * each gemv) */
 int mpres_batch_info(const mpres_batch_t *plan, double *mp_fmas, int *items, mpres_batch_tuning_t *used);
 int mpres_batch_destroy(mpres_batch_t *plan);
 

@@ -1316,8 +1316,10 @@ int mpres_batch_plan(mpres_ctx_t *c, const mpres_batch_problem_t *probs, int cou
     if (rc) return rc;
     BatchLayout lay;
     rc = batch_layout(probs, count, c->host.n, u.gemv_rows, lay, groups);
-    if (!rc && ws && groups && wsb < lay.ws_bytes)  // a workspace for fewer, larger items
+    if (!rc && ws && groups && wsb < lay.ws_bytes) {  // a workspace for fewer, larger items
+        groups = 0;
         rc = batch_layout(probs, count, c->host.n, u.gemv_rows, lay);
+    }
     if (rc) return fail(rc, "%s", lay.err.c_str());
     if (ws && wsb < lay.ws_bytes)
         return fail(MPRES_ERR_WORKSPACE, "workspace of %zu bytes, %zu needed", wsb, lay.ws_bytes);
@@ -1326,6 +1328,7 @@ int mpres_batch_plan(mpres_ctx_t *c, const mpres_batch_problem_t *probs, int cou
         hipError_t e = hipMalloc(&own, lay.ws_bytes);
         if (e != hipSuccess && groups) {  // likewise with the memory that there is
             (void)hipGetLastError();
+            groups = 0;
             rc = batch_layout(probs, count, c->host.n, u.gemv_rows, lay);
             if (rc) return fail(rc, "%s", lay.err.c_str());
             e = hipMalloc(&own, lay.ws_bytes);
@@ -1338,6 +1341,7 @@ int mpres_batch_plan(mpres_ctx_t *c, const mpres_batch_problem_t *probs, int cou
     b->count = (int)lay.items.size();
     b->fmas = lay.fmas;
     b->used = u;
+    if (groups) b->used.gemv_rows = 0;  // chosen for each gemv
     b->ws = own ? own : (char *)ws;
     b->own_ws = own != nullptr;
     *plan = b;

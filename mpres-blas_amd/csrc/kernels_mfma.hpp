@@ -141,7 +141,13 @@ k_mf_prescale(const DevConsts *__restrict__ C, int cnt, int JP, int k, int KP, i
         const int *dig = digits_of<N>(X, idx);
         for (int r = 0; r < N; r++) x[r] = dig[r];
     }
-    for (int r = 0; r < N; r++) x[r] = pos_reduce(x[r], C->m[r]);
+    bool out = false;  // residues outside [0, m) (Grp::reduce)
+#pragma unroll
+    for (int r = 0; r < N; r++) out |= (unsigned)x[r] >= (unsigned)C->m[r];
+    if (out) {
+#pragma unroll
+        for (int r = 0; r < N; r++) x[r] = modd((double)x[r], C->md[r], C->minv[r]);
+    }
     if (up.frac == 0 || -d > C->log2m + 1) {
         // zero, or truncated to zero (X < M < 2^(log2m + 1))
         for (int r = 0; r < N; r++) x[r] = 0;

@@ -19,52 +19,60 @@
 
 namespace mph {
 
-template <int N, int L>
+// the constants of a lane's one residue (Core::KC)
+template <int N, bool KC>
+struct CoreKept {};
+template <int N>
+struct CoreKept<N, true> {
+    double md, mv, rd, ru;
+    int mi, w, mrc[N - 1];
+    uint32_t wq;
+};
+template <int N, int L, bool KEEP = (N == L)>
 struct Core {
     static constexpr int R = N / L;
-    // One residue per lane (the inlined paths; at 8 moduli rounding runs on almost every step):
-    // the lane's constants are read once, by load(), and held in
-    // registers, so that no step waits on a reload of them. Otherwise they are read where used.
-    static constexpr bool KC = (R == 1);
-    static constexpr int KN = KC ? N - 1 : 1;
+    // KEEP: one residue per lane (the inlined paths; at 8 moduli rounding runs on almost every step): the
+    // lane's constants are read once, by load(), and held in registers, so that no step waits on a
+    // reload of them. Otherwise they are read where used, and the struct is small enough to go to the
+    // out-of-line functions in registers (through memory the finish of a precision form of 1024^2 entries
+    // over 16 moduli took 0.42 ms, now 0.37).
+    static constexpr bool KC = KEEP && R == 1;
     const DevConsts *__restrict__ C;
     const int *__restrict__ P2;
     int lane;
-    double kmd, kmv, krd, kru;
-    int kmi, kw, kmrc[KN];
-    uint32_t kwq;
+    CoreKept<N, KC> h;
     __device__ __forceinline__ void load() {
         if constexpr (KC) {
-            kmd = C->md[lane];
-            kmv = C->minv[lane];
-            krd = C->rrd[lane];
-            kru = C->rru[lane];
-            kmi = C->m[lane];
-            kw = C->w[lane];
-            kwq = C->wq[lane];
+            h.md = C->md[lane];
+            h.mv = C->minv[lane];
+            h.rd = C->rrd[lane];
+            h.ru = C->rru[lane];
+            h.mi = C->m[lane];
+            h.w = C->w[lane];
+            h.wq = C->wq[lane];
 #pragma unroll
-            for (int j = 0; j < KN; j++) kmrc[j] = C->mrcinv[j][lane];
+            for (int j = 0; j < N - 1; j++) h.mrc[j] = C->mrcinv[j][lane];
         }
     }
     __device__ __forceinline__ int ix(int r) const { return lane * R + r; }
     __device__ __forceinline__ double md(int r) const {
-        if constexpr (KC) return kmd;
+        if constexpr (KC) return h.md;
         else return C->md[ix(r)];
     }
     __device__ __forceinline__ double mv(int r) const {
-        if constexpr (KC) return kmv;
+        if constexpr (KC) return h.mv;
         else return C->minv[ix(r)];
     }
     __device__ __forceinline__ int mi(int r) const {
-        if constexpr (KC) return kmi;
+        if constexpr (KC) return h.mi;
         else return C->m[ix(r)];
     }
     __device__ __forceinline__ int w(int r) const {
-        if constexpr (KC) return kw;
+        if constexpr (KC) return h.w;
         else return C->w[ix(r)];
     }
     __device__ __forceinline__ uint32_t wq(int r) const {
-        if constexpr (KC) return kwq;
+        if constexpr (KC) return h.wq;
         else return C->wq[ix(r)];
     }
     // x_r times the weight w_r, mod m_r
@@ -77,16 +85,16 @@ struct Core {
         return mulmod_c((uint32_t)x, (uint32_t)p[0], (uint32_t)p[(size_t)(C->log2m + 1) * N], m);
     }
     __device__ __forceinline__ double rrd(int r) const {
-        if constexpr (KC) return krd;
+        if constexpr (KC) return h.rd;
         else return C->rrd[ix(r)];
     }
     __device__ __forceinline__ double rru(int r) const {
-        if constexpr (KC) return kru;
+        if constexpr (KC) return h.ru;
         else return C->rru[ix(r)];
     }
     // m_j^-1 mod m_i for j < i = ix(r) (the mixed-radix conversion's step j)
     __device__ __forceinline__ int mrc(int j, int r) const {
-        if constexpr (KC) return kmrc[j];
+        if constexpr (KC) return h.mrc[j];
         else return C->mrcinv[j][ix(r)];
     }
 };
@@ -183,8 +191,8 @@ __device__ __forceinline__ int bcast(int v, int src) {
 }
 
 // ---------------- mixed-radix conversion ----------------
-template <int N, int L, bool U>
-__device__ __forceinline__ void rns_mrc(Core<N, L> k, int *mr, const int *x) {
+template <int N, int L, bool U, bool KP>
+__device__ __forceinline__ void rns_mrc(Core<N, L, KP> k, int *mr, const int *x) {
     constexpr int R = N / L;
     loop<R, U>([&](int r) { mr[r] = x[r]; });
     loop<N - 1, U>([&](int j) {
@@ -205,15 +213,15 @@ __device__ __forceinline__ void rns_mrc(Core<N, L> k, int *mr, const int *x) {
         });
     });
 }
-template <int N, int L, bool U>
-__device__ __forceinline__ int rns_mrd(Core<N, L> k, const int *x) {
+template <int N, int L, bool U, bool KP>
+__device__ __forceinline__ int rns_mrd(Core<N, L, KP> k, const int *x) {
     constexpr int R = N / L;
     int mr[R];
     rns_mrc<N, L, U>(k, mr, x);
     return bcast<L>(mr[R - 1], L - 1);
 }
-template <int N, int L, bool U>
-__device__ __forceinline__ int rns_mrc_compare(Core<N, L> k, const int *x, const int *y) {
+template <int N, int L, bool U, bool KP>
+__device__ __forceinline__ int rns_mrc_compare(Core<N, L, KP> k, const int *x, const int *y) {
     constexpr int R = N / L;
     int mx[R], my[R];
     rns_mrc<N, L, U>(k, mx, x);
@@ -229,8 +237,8 @@ __device__ __forceinline__ int rns_mrc_compare(Core<N, L> k, const int *x, const
 // ---------------- interval evaluation ----------------
 constexpr int EVAL_MAX_ITER = 128;  // bound on the refinement loop; valid inputs need a handful
 
-template <int N, int L, bool U, bool FULL>
-__device__ __forceinline__ void rns_eval(Core<N, L> k, const int *x, Er &lo, Er &up, bool known_small) {
+template <int N, int L, bool U, bool FULL, bool KP>
+__device__ __forceinline__ void rns_eval(Core<N, L, KP> k, const int *x, Er &lo, Er &up, bool known_small) {
     constexpr int R = N / L;
     const DevConsts *C = k.C;
     int s[R];
@@ -293,8 +301,8 @@ __device__ __forceinline__ void rns_eval(Core<N, L> k, const int *x, Er &lo, Er 
 }
 
 // ---------------- power-of-two scaling ----------------
-template <int N, int L, bool U>
-__device__ __forceinline__ int rns_rank_full(Core<N, L> k, const int *x, const int *c) {
+template <int N, int L, bool U, bool KP>
+__device__ __forceinline__ int rns_rank_full(Core<N, L, KP> k, const int *x, const int *c) {
     constexpr int R = N / L;
     double fl[R], fu[R];
     loop<R, U>([&](int r) {
@@ -305,16 +313,16 @@ __device__ __forceinline__ int rns_rank_full(Core<N, L> k, const int *x, const i
     if (whl == whu) return (int)whl;
     return rns_mrd<N, L, U>(k, x) == 0 ? (int)whu : (int)whl;
 }
-template <int N, int L, bool U>
-__device__ __forceinline__ int rns_rank_fast(Core<N, L> k, const int *c) {
+template <int N, int L, bool U, bool KP>
+__device__ __forceinline__ int rns_rank_fast(Core<N, L, KP> k, const int *c) {
     constexpr int R = N / L;
     double fu[R];
     loop<R, U>([&](int r) { fu[r] = mul_ru((double)c[r], k.rru(r)); });
     return (int)psum_arr<N, L, true, U>(fu);
 }
 // y = (x - (X mod 2^j)) * 2^-j, given the rank kr of x
-template <int N, int L, bool U>
-__device__ __forceinline__ void rns_scale_step(Core<N, L> k, int *y, int kr, int j, const int *x, const int *c) {
+template <int N, int L, bool U, bool KP>
+__device__ __forceinline__ void rns_scale_step(Core<N, L, KP> k, int *y, int kr, int j, const int *x, const int *c) {
     constexpr int R = N / L;
     const uint32_t mask = (1u << j) - 1u;
     uint32_t part = 0;
@@ -329,13 +337,13 @@ __device__ __forceinline__ void rns_scale_step(Core<N, L> k, int *y, int kr, int
                         (uint32_t)k.mi(r));
     });
 }
-template <int N, int L, bool U>
-__device__ __forceinline__ void rns_xw(Core<N, L> k, int *c, const int *x) {
+template <int N, int L, bool U, bool KP>
+__device__ __forceinline__ void rns_xw(Core<N, L, KP> k, int *c, const int *x) {
     constexpr int R = N / L;
     loop<R, U>([&](int r) { c[r] = k.xw(x[r], r); });
 }
-template <int N, int L, bool U>
-__device__ __forceinline__ void rns_scale2pow(Core<N, L> k, int *x, unsigned D) {
+template <int N, int L, bool U, bool KP>
+__device__ __forceinline__ void rns_scale2pow(Core<N, L, KP> k, int *x, unsigned D) {
     constexpr int R = N / L;
     int c[R];
     int t = (int)(D / P2T);
@@ -360,8 +368,8 @@ __device__ __forceinline__ void rns_scale2pow(Core<N, L> k, int *x, unsigned D) 
 }
 
 // mp_round body: exp += bits, X = floor(X / 2^bits), fast re-evaluation
-template <int N, int L, bool U>
-__device__ __forceinline__ void mp_round_body(Core<N, L> k, int *d, int &exp, Er &ev0, Er &ev1) {
+template <int N, int L, bool U, bool KP>
+__device__ __forceinline__ void mp_round_body(Core<N, L, KP> k, int *d, int &exp, Er &ev0, Er &ev1) {
     const int bits = ev1.exp - k.C->mp_h + 1;
     exp += bits;
     rns_scale2pow<N, L, U>(k, d, (unsigned)bits);
@@ -369,8 +377,8 @@ __device__ __forceinline__ void mp_round_body(Core<N, L> k, int *d, int &exp, Er
 }
 
 // ---------------- out-of-line entry points (U = false) ----------------
-template <int N, int L, bool ELEM = false>  // ELEM: the element kernels' copy (Grp::round_here)
-__device__ __noinline__ void ool_round(Core<N, L> k, int *d, int *exp, Er *ev0, Er *ev1) {
+template <int N, int L, bool ELEM = false, bool KP>  // ELEM: the element kernels' copy (Grp::round_here)
+__device__ __noinline__ void ool_round(Core<N, L, KP> k, int *d, int *exp, Er *ev0, Er *ev1) {
     int e = *exp;
     Er a = *ev0, b = *ev1;
     mp_round_body<N, L, false>(k, d, e, a, b);
@@ -378,12 +386,12 @@ __device__ __noinline__ void ool_round(Core<N, L> k, int *d, int *exp, Er *ev0, 
     *ev0 = a;
     *ev1 = b;
 }
-template <int N, int L>
-__device__ __noinline__ int ool_mrc_compare(Core<N, L> k, const int *x, const int *y) {
+template <int N, int L, bool KP>
+__device__ __noinline__ int ool_mrc_compare(Core<N, L, KP> k, const int *x, const int *y) {
     return rns_mrc_compare<N, L, false>(k, x, y);
 }
-template <int N, int L>
-__device__ __noinline__ void ool_eval_full(Core<N, L> k, const int *x, Er *lo, Er *up, bool known_small) {
+template <int N, int L, bool KP>
+__device__ __noinline__ void ool_eval_full(Core<N, L, KP> k, const int *x, Er *lo, Er *up, bool known_small) {
     Er a, b;
     rns_eval<N, L, false, true>(k, x, a, b, known_small);
     *lo = a;

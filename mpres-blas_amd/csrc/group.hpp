@@ -227,16 +227,17 @@ __device__ __noinline__ void ool_reduce(const DevConsts *C, int *x, int *y, int 
 // 10^6 full products 8 lanes took 3.5 ms with it, one lane 0.66
 constexpr bool cold_round(int N, int L) { return (N == 16 && L <= 2) || (N > 16 && L == 1); }
 
-template <int N, int L>
+// INLINE: the rare paths inlined and unrolled
+template <int N, int L, bool INLINE = (N <= 8 || N == L)>
 struct Grp {
     static_assert(N % L == 0, "L must divide N");
     static_assert((L & (L - 1)) == 0 && L <= 32, "L must be a power of two <= 32");
     static constexpr int R = N / L;
-    static constexpr bool INL = (N <= 8 || R == 1);     // rare paths inlined and unrolled
+    static constexpr bool INL = INLINE;
     static constexpr bool CACHE = (L > 1 && R <= 8);    // per-lane moduli kept in registers
     static constexpr int CR = CACHE ? R : 1;
 
-    Core<N, L> k;
+    Core<N, L, INLINE && N == L> k;
     double cmd[CR], cmv[CR];
     int cmi[CR];
     uint32_t cmu[CR];

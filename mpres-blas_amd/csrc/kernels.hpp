@@ -47,8 +47,8 @@ constexpr int BLK = 256;
 constexpr int REDO = 2;  // sign of a workspace result whose chain the fixup kernel recomputes
 
 
-template <int N, int L>
-__device__ __forceinline__ void load_soa(const Grp<N, L> &g, MP<N / L> &a, const SoA &v, long long i) {
+template <int N, int L, bool I>
+__device__ __forceinline__ void load_soa(const Grp<N, L, I> &g, MP<N / L> &a, const SoA &v, long long i) {
     constexpr int R = N / L;
     const int *p = v.d + i * N + g.lane() * R;
 #pragma unroll
@@ -59,8 +59,8 @@ __device__ __forceinline__ void load_soa(const Grp<N, L> &g, MP<N / L> &a, const
     a.ev0 = Er{lo.frac, (int)lo.exp};
     a.ev1 = Er{up.frac, (int)up.exp};
 }
-template <int N, int L>
-__device__ __forceinline__ void store_soa(const Grp<N, L> &g, const MP<N / L> &a, const SoA &v, long long i) {
+template <int N, int L, bool I>
+__device__ __forceinline__ void store_soa(const Grp<N, L, I> &g, const MP<N / L> &a, const SoA &v, long long i) {
     constexpr int R = N / L;
     int *p = v.d + i * N + g.lane() * R;
 #pragma unroll
@@ -72,8 +72,8 @@ __device__ __forceinline__ void store_soa(const Grp<N, L> &g, const MP<N / L> &a
         v.ev[i + v.len] = ErMem{a.ev1.frac, (long long)a.ev1.exp};
     }
 }
-template <int N, int L>
-__device__ __forceinline__ void load_aos(const Grp<N, L> &g, MP<N / L> &a, const AoSRef<N> &v, long long i) {
+template <int N, int L, bool I>
+__device__ __forceinline__ void load_aos(const Grp<N, L, I> &g, MP<N / L> &a, const AoSRef<N> &v, long long i) {
     constexpr int R = N / L;
     const int *p = v.digits(i) + g.lane() * R;
 #pragma unroll
@@ -85,8 +85,8 @@ __device__ __forceinline__ void load_aos(const Grp<N, L> &g, MP<N / L> &a, const
     a.ev0 = Er{lo.frac, (int)lo.exp};
     a.ev1 = Er{up.frac, (int)up.exp};
 }
-template <int N, int L>
-__device__ __forceinline__ void store_aos(const Grp<N, L> &g, const MP<N / L> &a, const AoSRef<N> &v, long long i) {
+template <int N, int L, bool I>
+__device__ __forceinline__ void store_aos(const Grp<N, L, I> &g, const MP<N / L> &a, const AoSRef<N> &v, long long i) {
     constexpr int R = N / L;
     int *p = v.digits(i) + g.lane() * R;
 #pragma unroll

@@ -33,8 +33,8 @@ __device__ __forceinline__ void wg_sync() {
 
 // k_tree's halving tree over nb blocks of b partials each (block q at part[q * b]), all
 // blocks level by level: for s = nextPow2(b)/2 .. 1: p[t] = p[t] + p[t + s] for t < s, t + s < b
-template <int N, int L>
-__device__ void batch_tree(const Grp<N, L> &g, AoSRef<N> part, long long nb, int b) {
+template <int N, int L, bool I>
+__device__ void batch_tree(const Grp<N, L, I> &g, AoSRef<N> part, long long nb, int b) {
     constexpr int W = BLK / L;
     const int gl = threadIdx.x / L;
     unsigned p2 = 1;
@@ -57,8 +57,8 @@ __device__ void batch_tree(const Grp<N, L> &g, AoSRef<N> part, long long nb, int
 }
 
 // dot: scratch = grid3 * block3 partials, then block3 second-pass partials
-template <int N, int L>
-__device__ void batch_dot(const Grp<N, L> &g, const BatchItem &it, char *ws) {
+template <int N, int L, bool I>
+__device__ void batch_dot(const Grp<N, L, I> &g, const BatchItem &it, char *ws) {
     constexpr int W = BLK / L;
     const int gl = threadIdx.x / L;
     const SoA x = rd(it.x), y = rd(it.y);
@@ -94,8 +94,8 @@ __device__ void batch_dot(const Grp<N, L> &g, const BatchItem &it, char *ws) {
 }
 
 // gemv rows [r0, r1): scratch = bx (lx numbers), then (r1 - r0) * block3 partials
-template <int N, int L, bool TRANS>
-__device__ void batch_gemv(const Grp<N, L> &g, const BatchItem &it, char *ws) {
+template <int N, int L, bool TRANS, bool I>
+__device__ void batch_gemv(const Grp<N, L, I> &g, const BatchItem &it, char *ws) {
     constexpr int W = BLK / L;
     const int gl = threadIdx.x / L;
     const SoA alpha = rd(it.alpha), A = rd(it.A), x = rd(it.x), beta = rd(it.beta), y = rd(it.y);
@@ -148,7 +148,10 @@ template <int N, int L>
 __global__ __launch_bounds__(BLK) void k_batch(const DevConsts *__restrict__ C, const BatchItem *__restrict__ items,
                                                int count, int *queue, char *ws) {
     __shared__ int next;
-    Grp<N, L> g(C);
+    // over 16 and 32 moduli the rare paths stay out of line also with one residue a lane: inlined in
+    // every phase they cost half the waves (212 bits, 16 lanes, 4 workgroups a CU: 4096 dots and gemvs 31.9
+    // ms, out of line 21.4; 1024 of them, which leave the chip half empty, 9.8 and 13.6)
+    const Grp<N, L, (N <= 8)> g(C);
     for (;;) {
         if (threadIdx.x == 0) next = atomicAdd(queue, 1);
         __syncthreads();

@@ -76,9 +76,11 @@ const Ops *find_ops(int n, int L) { return find_variant(n, L); }
 // mpres-blas_amd/tuning/lanes_gfx950.json): a call of size <= bound[i] uses lanes[i], a
 // larger one the last entry. That table is of operands that are doubles; the axpy, element, gemm
 // and SpMV entries over 16 and 32 moduli weigh full operands, whose every product rounds, as
-// well: with one lane a number (two at 16 moduli up to 65536) they round positionally, axpy_v2 of
-// 120000 numbers of 212 bits 0.058 ms against 0.32 with 4 lanes (doubles 0.013 and 0.011), and
-// with one modulus a lane the rounding is inlined (20000 numbers 0.033 against 0.11 ms). Installed at context creation for these sets; mpres_set_lanes
+// well: with one lane a number, or two for calls of middling size, they round positionally, and with one
+// modulus a lane the rounding is inlined. axpy_v2 in us, doubles and full operands: 212 bits, 120000
+// numbers, one lane 13 and 60, 4 lanes 13 and 310; 20000 numbers, 16 lanes 5 and 33, 4 lanes 5 and 110; 424
+// bits, 30000 numbers, two lanes 8 and 108, 8 lanes 7 and 185, one lane 11 and 108; 250000 numbers, one lane
+// 45 and 332, 8 lanes 37 and 1473. Installed at context creation for these sets; mpres_set_lanes
 // replaces an operation's table by a fixed choice, mpres_set_lanes(op, 0) restores it.
 struct BuiltinLanes {
     const char *set;
@@ -100,7 +102,7 @@ const BuiltinLanes kBuiltinLanes[] = {
     {"16_4double", OP_SPMV, 1, {1000000LL}, {16}},
     {"16_4double", OP_ELEM, 2, {32768LL, 1048576LL}, {16, 1}},
     {"32_8double", OP_DOT, 4, {16384LL, 262144LL, 4194304LL, 16777216LL}, {32, 8, 8, 8}},
-    {"32_8double", OP_AXPY, 2, {16384LL, 16777216LL}, {32, 1}},
+    {"32_8double", OP_AXPY, 3, {16384LL, 98304LL, 16777216LL}, {32, 2, 1}},
     {"32_8double", OP_GEMV, 4, {16384LL, 262144LL, 4194304LL, 16777216LL}, {32, 4, 8, 8}},
     {"32_8double", OP_GEMM, 4, {741455LL, 5931641LL, 47453132LL, 134217728LL}, {8, 8, 8, 8}},
     {"32_8double", OP_SPMV, 1, {1000000LL}, {32}},
@@ -600,13 +602,22 @@ int mpres_array_to_aos(mpres_ctx_t *c, void *dst, const mp_array_t *src, int cou
     return MPRES_OK;
 }
 
-// The variant of an element-wise call. Over 32 moduli a sum, which seldom rounds, keeps 8 lanes
-// a number where the built-in table gives one for the products (a sum of 10^6 in 0.135 ms with 8
-// lanes, 0.193 ms with one; a product of full operands in 4.6 and 0.66 ms).
+// The variant of an element-wise call, where the built-in table is in use: the calls of mp_float_t arrays
+// read whole records, which one lane a number does badly while nothing rounds. In us, doubles and full
+// operands: 212 bits, products of 250000, two lanes 17 and 74, one lane 22 and 58, 4 lanes 14 and 340; sums of
+// 10^6, two lanes 88 and 285, one lane 104 and 232, 4 lanes 80 and 470; 424 bits, products of 60000, two
+// lanes 8 and 107, one lane 10 and 99, 8 lanes 7 and 312; of 10^6, one lane 146 and 646, two lanes 107 and
+// 1147, 8 lanes 105 and 4517. Sums over 32 moduli, which seldom round, keep 8 lanes (10^6 0.135 ms, one
+// lane 0.18).
 static const Ops *elem_ops(const mpres_ctx *c, int op, int count) {
     const Ops *o = sized(c, OP_ELEM, count);
+    if (!c->lt[OP_ELEM].builtin || c->host.n == 8) return o;
     const bool sum = op == 0 || op == 1 || op == 4;
-    return c->host.n == 32 && sum && o->L == 1 && c->lt[OP_ELEM].builtin ? find_ops(32, 8) : o;
+    int L = o->L;
+    if (c->host.n == 16 && count > 16384) L = 2;
+    if (c->host.n == 32 && sum) L = 8;
+    if (c->host.n == 32 && !sum && count > 16384 && count <= 524288) L = 2;
+    return L == o->L ? o : find_ops(c->host.n, L);
 }
 
 int mpres_elementwise(mpres_ctx_t *c, int op, int count, const void *x, const void *y, void *r, void *st) {

@@ -224,8 +224,8 @@ __device__ __noinline__ void ool_reduce(const DevConsts *C, int *x, int *y, int 
 
 // element kernels that round in a function of their own (Grp::round_fails). With more lanes a
 // number that function, run by one lane of the group, leaves the others idle: over 32 moduli and
-// 10^6 full products 8 lanes took 3.5 ms with it, one lane 0.66
-constexpr bool cold_round(int N, int L) { return (N == 16 && L <= 2) || (N > 16 && L == 1); }
+// 10^6 full products 8 lanes took 3.5 ms with it, two 1.15 and one 0.65 (8 lanes without it 4.5)
+constexpr bool cold_round(int N, int L) { return N > 8 && L <= 2; }
 
 // INLINE: the rare paths inlined and unrolled
 template <int N, int L, bool INLINE = (N <= 8 || N == L)>

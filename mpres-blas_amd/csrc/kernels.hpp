@@ -33,7 +33,7 @@
 namespace mph {
 
 constexpr int BLK = 256;
-// Element kernels with one lane per number over 16 and 32 moduli are held to three (two) waves
+// Element kernels with one lane per number (or two, cold_round) over 16 and 32 moduli are held to three (two) waves
 // per SIMD, which is what the positional rounding needs to keep its integers in registers: inlined
 // in the kernel (ELEM_WAVES), or in the function that does a number again (COLD_WAVES,
 // Grp::round_fails).

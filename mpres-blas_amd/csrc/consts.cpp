@@ -75,6 +75,12 @@ static double emu_div_ru(double a, double b) {
 bool compute_consts(const ModuliSet &s, DevConsts &c, std::vector<int> &pow2) {
     std::memset(&c, 0, sizeof c);
     const int n = s.n;
+    // What the integer arithmetic rests on: 3 m below 2^32 (mulmod_i), which with at most 32 moduli also
+    // keeps the columns of pos_from_digits below 2^64; one bit length for the moduli of a set
+    if (n < 1 || n > MAXN) return false;
+    for (int i = 0; i < n; i++)
+        if (s.m[i] < 3 || 3LL * s.m[i] >= 1LL << 32 || __builtin_clz((unsigned)s.m[i]) != __builtin_clz((unsigned)s.m[0]))
+            return false;
     c.n = n;
     c.log2m = s.log2m;
     for (int i = 0; i < n; i++) {
@@ -84,7 +90,6 @@ bool compute_consts(const ModuliSet &s, DevConsts &c, std::vector<int> &pow2) {
     }
     c.mus = 31 - __builtin_clz((unsigned)s.m[0]);
     for (int i = 0; i < n; i++) {
-        if (31 - __builtin_clz((unsigned)s.m[i]) != c.mus) return false;  // moduli of one set have one bit length
         c.mu[i] = (uint32_t)(((uint64_t)1 << (c.mus + 32)) / (uint32_t)s.m[i]);
     }
     // M in 32-bit limbs

@@ -83,8 +83,9 @@ __device__ __forceinline__ int pos_reduce(int d, int m) {
 // The integer of residues (any int from 0 of the class): X = sum c_i M/m_i - rank M with c_i = |x_i w_i| mod m_i, its low WX
 // words. NORM: X / M below 2^-40, and rank the nearest integer of sum c_i / m_i; otherwise any
 // X < M (WX = N: all of it): rank is the whole part of a sum that may be off by 2^-40, so the
-// result is brought into [0, M). Columns of 28-bit limbs in 64 bits: N products below 2^59 and a carry
-// below 2^37 (v_mad_u64_u32 runs at full rate); the rank's multiple of 2^K - M joins the column.
+// result is brought into [0, M). Columns of 28-bit limbs in 64 bits: at most 32 products
+// below 1.43e9 2^28 (compute_consts), the rank's multiple of 2^K - M, below 2^33, and a carry below 2^36
+// stay below 2^63.5.
 template <int N, int WX, bool NORM>
 __device__ __forceinline__ void pos_from_digits(const DevConsts *__restrict__ C, const int *d, uint32_t *x) {
     constexpr int LN = (32 * WX + 27) / 28;

@@ -230,10 +230,16 @@ struct WsUse {
         return MPRES_OK;
     }
     // as get, for a call that runs faster with `full` bytes but does with `need`: *have tells
-    // whether there are `full` (a caller's smaller workspace, or a pool that cannot grow so far,
-    // is taken as it is)
+    // whether there are `full` (a caller's smaller workspace, or a pool that cannot grow so far, is
+    // taken as it is; so is a pool that would do while the stream is captured, which a growth would end)
     int get2(void *ws, size_t ws_bytes, size_t need, size_t full, char **out, bool *have) {
-        *have = full > need && (ws ? ws_bytes >= full : get(nullptr, 0, full, out) == MPRES_OK);
+        bool grow = true;
+        if (!ws && c->ws_bytes >= need && c->ws_bytes < full) {
+            hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+            if (hipStreamIsCapturing(st, &status) != hipSuccess) (void)hipGetLastError();
+            grow = status == hipStreamCaptureStatusNone;
+        }
+        *have = full > need && (ws ? ws_bytes >= full : grow && get(nullptr, 0, full, out) == MPRES_OK);
         if (*have && !ws) return MPRES_OK;
         if (!ws) (void)hipGetLastError();
         return get(ws, ws_bytes, need, out);

@@ -161,17 +161,6 @@ MPH_HD void big_add_u32(Big<W> &a, uint32_t v) {
         carry = t >> 32;
     }
 }
-// a = a * m + c
-template <int W>
-MPH_HD void big_mul_add_u32(Big<W> &a, uint32_t m, uint32_t c) {
-    uint64_t carry = c;
-#pragma unroll
-    for (int i = 0; i < W; i++) {
-        const uint64_t t = (uint64_t)a.l[i] * m + carry;
-        a.l[i] = (uint32_t)t;
-        carry = t >> 32;
-    }
-}
 // a * b, exactly
 template <int A, int B>
 MPH_HD Big<A + B> big_mul(const Big<A> &a, const Big<B> &b) {

@@ -205,13 +205,21 @@ int mpres_dot_noalloc(mpres_ctx_t *ctx, int n, const mp_array_t *x, int incx, co
 int mpres_axpy(mpres_ctx_t *ctx, int n, const mp_array_t *alpha, const mp_array_t *x, int incx, mp_array_t *y,
                int incy, void *stream);
 /* y = alpha*op(A)*x + beta*y ; cuda::mp_gemv<gridDim1,blockDim1,gridDim2,blockDim3>, src/blas/gemv.cuh:150-268.
- * The sum order of each output is fixed by blockDim3. */
+ * The sum order of each output is fixed by blockDim3.
+ * Workspace: alpha * x, the partial sums and the row sums as mp_float_t, over 16 and 32 moduli without
+ * transposition x's residues and the rows' exponents, and over 8 moduli alpha * x once more as positional
+ * records (32 bytes a number). mpres_gemv_workspace gives all of it; a buffer without room for the records is
+ * accepted, and alpha * x is then converted for every product again (ws NULL: the context's pool). */
 size_t mpres_gemv_workspace(const mpres_ctx_t *ctx, int trans, int m, int n, int block3);
 int mpres_gemv(mpres_ctx_t *ctx, int trans, int m, int n, const mp_array_t *alpha, const mp_array_t *A, int lda,
                const mp_array_t *x, int incx, const mp_array_t *beta, mp_array_t *y, int incy, int block3, void *ws,
                size_t ws_bytes, void *stream);
 /* C = alpha*A*B + beta*C ; cuda::mp_gemm<...>, src/blas/gemm.cuh:69-167 (no-trans only, as the reference).
- * Workspace: the m*n dot-product sums as mp_float_t (ws NULL: the context's pool).
+ * Workspace: the m*n dot-product sums as mp_float_t, over 16 and 32 moduli the residue planes, and after
+ * them what makes the call faster: over 8 moduli A and B as positional records (32 bytes a number), over
+ * 16 and 32 with k >= 16 the bounds of the scalar chains (20 bytes a number of A and B). mpres_gemm_workspace
+ * gives all of it; a buffer without room for the last part is accepted, and the call then works from A and B
+ * as they lie (ws NULL: the context's pool).
  * A->digits and B->digits must be 16-byte aligned (device allocations are), else MPRES_ERR_ARG. */
 size_t mpres_gemm_workspace(const mpres_ctx_t *ctx, int m, int n, int k);
 int mpres_gemm(mpres_ctx_t *ctx, int transa, int transb, int m, int n, int k, const mp_array_t *alpha,
@@ -389,7 +397,7 @@ int mpres_cg_csr(mpres_ctx_t *ctx, int n, const csr_t *A, const void *b, double 
                  size_t ws_bytes, void *stream);
 
 /* cuda::mp_gemm(transa,transb,...), src/blas/v2/gemm_v2.cuh:55-81.
- * Workspace: the m*n sums, as for mpres_gemm (mpres_gemm_workspace). */
+ * Workspace: as for mpres_gemm (mpres_gemm_workspace). */
 int mpres_gemm_v2(mpres_ctx_t *ctx, int transa, int transb, int m, int n, int k, const void *alpha, const void *A,
                   int lda, const void *B, int ldb, const void *beta, void *C, int ldc, void *ws, size_t ws_bytes,
                   void *stream);
@@ -488,7 +496,12 @@ int mpres_profile_read(mpres_ctx_t *ctx, int op, double *ms, long *launches, int
  * The built-in choice for the 8_2double, 16_4double and 32_8double sets is a table by call
  * size measured on MI355X (mpres-blas_amd/tuning/lanes_gfx950.json) for elementwise, dot,
  * gemv, gemm, spmv and axpy; mpres_set_lanes with a nonzero count replaces it by that fixed count,
- * with 0 restores it. mpres_get_lanes: the choice without a table. */
+ * with 0 restores it. mpres_get_lanes: the choice without a table.
+ * Over 8 moduli the main kernels of gemv, gemm and dots of 8 or more terms a chain run on positional
+ * integers, a lane or four a chain by the number of chains; the lanes of those operations act on their other
+ * kernels (scalings, trees, epilogue, fixup, shorter dots). Over 16 and 32 moduli the built-in choice of
+ * elementwise calls also looks at the operation: sums and products may run on fewer lanes than the table
+ * says. */
 int mpres_lanes_supported(const mpres_ctx_t *ctx, int lanes);
 int mpres_set_lanes(mpres_ctx_t *ctx, int op, int lanes);
 int mpres_get_lanes(const mpres_ctx_t *ctx, int op);  /* lanes in use, or a negative error */
@@ -499,7 +512,7 @@ int mpres_get_lanes(const mpres_ctx_t *ctx, int op);  /* lanes in use, or a nega
  * Size: the call's multiply-accumulate count (dot and axpy n, gemv m n, gemm and the
  * precision form m n k), the row count for SpMV, the element count for mpres_elementwise.
  * No reference counterpart; results do not depend on it. mpres-blas_amd/lanes_tune.py
- * measures a table. mpres_get_lanes_for: the lanes a call of that size uses. */
+ * measures a table. mpres_get_lanes_for: the table's lanes for a call of that size. */
 #define MPRES_LANES_TABLE_MAX 8
 int mpres_set_lanes_table(mpres_ctx_t *ctx, int op, int count, const long long *bounds, const int *lanes);
 int mpres_get_lanes_for(const mpres_ctx_t *ctx, int op, long long size);

@@ -613,14 +613,15 @@ int mpres_array_to_aos(mpres_ctx_t *c, void *dst, const mp_array_t *src, int cou
 // operands: 212 bits, products of 250000, two lanes 17 and 74, one lane 22 and 58, 4 lanes 14 and 340; sums of
 // 10^6, two lanes 88 and 285, one lane 104 and 232, 4 lanes 80 and 470; 424 bits, products of 60000, two
 // lanes 8 and 107, one lane 10 and 99, 8 lanes 7 and 312; of 10^6, one lane 146 and 646, two lanes 107 and
-// 1147, 8 lanes 105 and 4517. Sums over 32 moduli, which seldom round, keep 8 lanes (10^6 0.135 ms, one
-// lane 0.18).
+// 1147, 8 lanes 105 and 4517. Up to 24576 numbers of 212 bits keep 16 lanes: products of 20000, 16 lanes 5
+// and 17, two lanes 4 and 19; sums, 16 lanes 5 and 10, two lanes 5 and 23. Sums over 32 moduli, which seldom
+// round, keep 8 lanes (10^6 0.135 ms, one lane 0.18).
 static const Ops *elem_ops(const mpres_ctx *c, int op, int count) {
     const Ops *o = sized(c, OP_ELEM, count);
     if (!c->lt[OP_ELEM].builtin || c->host.n == 8) return o;
     const bool sum = op == 0 || op == 1 || op == 4;
     int L = o->L;
-    if (c->host.n == 16 && count > 16384) L = 2;
+    if (c->host.n == 16 && count > 24576) L = 2;
     if (c->host.n == 32 && sum) L = 8;
     if (c->host.n == 32 && !sum && count > 16384 && count <= 524288) L = 2;
     return L == o->L ? o : find_ops(c->host.n, L);
@@ -692,8 +693,9 @@ size_t mpres_dot_workspace(const mpres_ctx_t *c, int n, int g3, int b3) {
 }
 
 // Terms per chain from which the positional chains are used: converting a sum back and evaluating
-// it costs about as much as 6 terms of the residue chain (8 moduli, 256 x 64 chains: 4 terms
-// 31 us against 23 us, 16 terms about 50 us against 95 us, 1024 terms 1.50 ms against 6.12 ms).
+// it costs about as much as 6 terms of the residue chain. Whole calls over 8 moduli with 256 x 64 chains,
+// residue and positional chains: 8 terms 96 and 100 us, 16 terms 142 and 113 us, 64 terms 411 and 170 us, 1024
+// terms 6.08 and 1.18 ms.
 constexpr long long POS_DOT_TERMS = 8;
 static int dot_common(mpres_ctx_t *c, WsUse &wu, int mode, int n, SoA xs, int incx, SoA ys, int incy,
                       const char *xa, const char *ya, int g3, int b3, void *ws, size_t wsb, hipStream_t st,

@@ -77,10 +77,11 @@ const Ops *find_ops(int n, int L) { return find_variant(n, L); }
 // larger one the last entry. That table is of operands that are doubles; the axpy, element, gemm
 // and SpMV entries over 16 and 32 moduli weigh full operands, whose every product rounds, as
 // well: with one lane a number, or two for calls of middling size, they round positionally, and with one
-// modulus a lane the rounding is inlined. axpy_v2 in us, doubles and full operands: 212 bits, 120000
-// numbers, one lane 13 and 60, 4 lanes 13 and 310; 20000 numbers, 16 lanes 5 and 33, 4 lanes 5 and 110; 424
-// bits, 30000 numbers, two lanes 8 and 108, 8 lanes 7 and 185, one lane 11 and 108; 250000 numbers, one lane
-// 45 and 332, 8 lanes 37 and 1473. Installed at context creation for these sets; mpres_set_lanes
+// modulus a lane the rounding is inlined. axpy in us, doubles and full operands, one, two and 4 (8) lanes:
+// 212 bits, 150000 numbers 15 and 59, 12 and 91, 13 and 308; 500000, 37 and 147, 35 and 236, 37 and 870; 10^6,
+// 64 and 266, 66 and 433, 74 and 2227; 424 bits, 100000 numbers 21 and 154, 19 and 253, 17 and 686; 500000, 80
+// and 526, 71 and 923, 67 and 2910; 10^6, 155 and 1029, 172 and 1791, 175 and 7484. Two lanes up to the sizes
+// where one is as fast for doubles. Installed at context creation for these sets; mpres_set_lanes
 // replaces an operation's table by a fixed choice, mpres_set_lanes(op, 0) restores it.
 struct BuiltinLanes {
     const char *set;
@@ -96,13 +97,13 @@ const BuiltinLanes kBuiltinLanes[] = {
     {"8_2double", OP_SPMV, 3, {31622LL, 316227LL, 1000000LL}, {8, 8, 8}},
     {"8_2double", OP_ELEM, 3, {16384LL, 262144LL, 1048576LL}, {8, 2, 2}},
     {"16_4double", OP_DOT, 4, {16384LL, 262144LL, 4194304LL, 16777216LL}, {16, 16, 4, 4}},
-    {"16_4double", OP_AXPY, 3, {24576LL, 65536LL, 16777216LL}, {16, 2, 1}},
+    {"16_4double", OP_AXPY, 3, {24576LL, 393216LL, 16777216LL}, {16, 2, 1}},
     {"16_4double", OP_GEMV, 4, {16384LL, 262144LL, 4194304LL, 16777216LL}, {16, 16, 16, 16}},
     {"16_4double", OP_GEMM, 1, {134217728LL}, {16}},
     {"16_4double", OP_SPMV, 1, {1000000LL}, {16}},
     {"16_4double", OP_ELEM, 2, {32768LL, 1048576LL}, {16, 1}},
     {"32_8double", OP_DOT, 4, {16384LL, 262144LL, 4194304LL, 16777216LL}, {32, 8, 8, 8}},
-    {"32_8double", OP_AXPY, 3, {16384LL, 98304LL, 16777216LL}, {32, 2, 1}},
+    {"32_8double", OP_AXPY, 3, {16384LL, 524288LL, 16777216LL}, {32, 2, 1}},
     {"32_8double", OP_GEMV, 4, {16384LL, 262144LL, 4194304LL, 16777216LL}, {32, 4, 8, 8}},
     {"32_8double", OP_GEMM, 4, {741455LL, 5931641LL, 47453132LL, 134217728LL}, {8, 8, 8, 8}},
     {"32_8double", OP_SPMV, 1, {1000000LL}, {32}},
@@ -612,8 +613,8 @@ int mpres_array_to_aos(mpres_ctx_t *c, void *dst, const mp_array_t *src, int cou
 // read whole records, which one lane a number does badly while nothing rounds. In us, doubles and full
 // operands: 212 bits, products of 250000, two lanes 17 and 74, one lane 22 and 58, 4 lanes 14 and 340; sums of
 // 10^6, two lanes 88 and 285, one lane 104 and 232, 4 lanes 80 and 470; 424 bits, products of 60000, two
-// lanes 8 and 107, one lane 10 and 99, 8 lanes 7 and 312; of 10^6, one lane 146 and 646, two lanes 107 and
-// 1147, 8 lanes 105 and 4517. Up to 24576 numbers of 212 bits keep 16 lanes: products of 20000, 16 lanes 5
+// lanes 8 and 107, one lane 10 and 99, 8 lanes 7 and 312; of 10^6, two lanes 106 and 1152, 8 lanes
+// 104 and 4518, one lane 147 and 643. Up to 24576 numbers of 212 bits keep 16 lanes: products of 20000, 16 lanes 5
 // and 17, two lanes 4 and 19; sums, 16 lanes 5 and 10, two lanes 5 and 23. Sums over 32 moduli, which seldom
 // round, keep 8 lanes (10^6 0.135 ms, one lane 0.18).
 static const Ops *elem_ops(const mpres_ctx *c, int op, int count) {
@@ -623,7 +624,7 @@ static const Ops *elem_ops(const mpres_ctx *c, int op, int count) {
     int L = o->L;
     if (c->host.n == 16 && count > 24576) L = 2;
     if (c->host.n == 32 && sum) L = 8;
-    if (c->host.n == 32 && !sum && count > 16384 && count <= 524288) L = 2;
+    if (c->host.n == 32 && !sum && count > 16384) L = 2;
     return L == o->L ? o : find_ops(c->host.n, L);
 }
 

@@ -18,8 +18,8 @@
 // every case of the reference arithmetic. Both kernels run the identical
 // sequence of operations, so the result does not depend on which one
 // finished a chain. Over 8 moduli rounding is the common case: the main
-// kernels there are the positional ones (kernels_pos.hpp), and the single full kernel
-// for the short chains of a dot.
+// kernels of gemv, gemm and long dots are the positional ones there (kernels_pos.hpp), with the
+// fixup kernel for what they mark; short chains of a dot and SpMV run the single full kernel.
 #pragma once
 
 #include <hip/hip_runtime.h>

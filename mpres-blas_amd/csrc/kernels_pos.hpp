@@ -5,8 +5,8 @@
 // operands, which is most of a step's work, runs in parallel, and the products reach the other
 // lanes by quad permutations (DPP, no LDS). That serves calls with few chains. With G = 1 a
 // lane does a whole chain, for calls with enough of them to fill the chip.
-// What bounds them is the serial chain: about 290 vector instructions a sum and 190 a product,
-// issued by one or two waves per SIMD. Against the residue chains over 8 moduli: dot of 2^24
+// What bounds them is the serial chain: 1560 vector instructions a wave for four terms of its quads
+// (a product a lane, four sums), issued by one or two waves per SIMD. Against the residue chains over 8 moduli: dot of 2^24
 // terms in 256 x 64 chains 6.12 -> 1.18 ms, A^T x of a 1501 x 777 matrix in 24864 chains
 // 697 -> 150 us.
 #pragma once

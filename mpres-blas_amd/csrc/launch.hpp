@@ -169,7 +169,8 @@ struct Launch {
     // and pre-scaled residues of bx), 1 main kernel (split form: the residues), 2 split
     // form: the scalar chains (independent of pass 1, so a caller may run the two on two
     // streams), 3 split form: the residues moved to the chains' results, 4 the fixup of the
-    // partials still marked. Over 8 moduli the main kernel is the positional one (PosOps). aux: the split form's bxp (N*n ints), EA (m ints), EB (1 int).
+    // partials still marked. Over 8 moduli the main kernel is the positional one (PosOps). aux: the
+    // split form's bxp (N*n ints), EA (m ints), EB (1 int).
     static bool gemv_split(bool trans, int b3) { return SPLIT && !trans && b3 <= 65535; }
     static size_t gemv_aux(bool trans, int m, int n) {
         return (SPLIT && !trans) ? 4 * ((size_t)N * n + m + 1) : 0;
@@ -238,7 +239,8 @@ struct Launch {
     // gemm passes. Over 16 and 32 moduli (split form, see kernels.hpp):
     //   0 exponent minima and the int8 limb planes of the pre-scaled residues, 1 scalar chains,
     //   2 residue products (INT8 MFMA) and digits, 3 fixup of the marked chains, 4 epilogue.
-    // Over 8 moduli the sums are the positional kernel's (PosOps): 3 fixup, 4 epilogue. bits: bit length of the largest modulus.
+    // Over 8 moduli the sums are the positional kernel's (PosOps): 3 fixup, 4 epilogue. bits: bit
+    // length of the largest modulus.
     // ws: m*n sums, then (split form) the residue sums S (N*m*n ints), the minima (m + n
     // ints) and the limb planes of op(A) and op(B).
     static constexpr int GEMM_NL = 5;  // limbs per residue reserved (moduli below 2^35)
@@ -306,7 +308,8 @@ struct Launch {
                                        m, n, k, A, lda, B, ldb, (const ChainOp *)pa, (const int *)ea,
                                        (const ChainOp *)pb, (const int *)eb, sums);
             } else if (pass == 1) {
-                // a workspace without room for the operands, or short chains: no transposes and element offsets below 2^28: the specialised chain kernel
+                // a workspace without room for the operands, or short chains; without transposes and
+                // with element offsets below 2^28 the specialised chain kernel
                 if constexpr (std::is_same<VM, SoA>::value) {
                     if (ta == 0 && tb == 0 && (long long)lda * k <= (1LL << 28) && (long long)ldb * n <= (1LL << 28)) {
                         if (m % 64 == 0)

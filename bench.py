@@ -527,7 +527,9 @@ def plain_lines(mp, threads, cpu=True):
         err = rel_err(exact_value(ctx.array_to_host(r, 1)[0], m_), want)
         b = 2.0 * n * S
         line = {"op": "mp_dot", "moduli_set": "8_2double", "bits": ctx.precision, "n": n,
-                "order": "gridDim3=256, blockDim3=64", "lanes_per_number": L.mpres_get_lanes_for(ctx.h, mp.K_DOT, n),
+                "order": "gridDim3=256, blockDim3=64",
+                # from 8 terms a chain on: positional integers, four lanes a chain
+                "lanes_per_number": 4 if n >= 8 * 256 * 64 else L.mpres_get_lanes_for(ctx.h, mp.K_DOT, n),
                 "ms": ms, "mpfma_per_s": n / (ms / 1e3),
                 "bytes": b, "gbs": b / (ms / 1e3) / 1e9, "hbm_frac": b / (ms / 1e3) / 1e9 / HBM_PEAK_GBS,
                 "max_rel_err": err}

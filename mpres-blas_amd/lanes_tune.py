@@ -9,7 +9,9 @@ compiled lane count on synthetic inputs (u 2^e, e in [-20, 20]; gemv and gemm wi
 beta = 0, so that repeated calls do the same work) and keeps the fastest. The table it writes (one entry per size, the bound of each bucket
 halfway, geometrically, to the next size) plays the part of the reference's
 compile-time launch constants (src/kernel_config.cuh), chosen by measurement
-per size; load() installs it in a context.
+per size; load() installs it in a context. Over 8 moduli the main kernels of
+gemv, gemm and long dots are positional and use lanes of their own: what is timed
+there is the lanes of their other kernels.
 
     python lanes_tune.py [--sets 8_2double,16_4double,32_8double] [--out tuning/lanes_gfx950.json]
 """
